@@ -194,8 +194,9 @@ class HipRealizerBridge:
                   trans_b: bool = False, in_dtype: str = "float32", out_dtype: Optional[str] = None,
                   bias: Optional[int] = None, round_out: bool = False, act: int = N.ACT_NONE,
                   residual: Optional[int] = None, a_dtype: Optional[str] = None,
-                  b_dtype: Optional[str] = None) -> int:
-        """bg_matmul_ex; with ``residual`` (f32 [batch, m, n] added after
+                  b_dtype: Optional[str] = None, f32_unsplit: bool = False) -> int:
+        """bg_matmul_ex; ``f32_unsplit`` forms every float32 product by a
+        float32 matrix instruction (BG_MATMUL_F32_UNSPLIT); with ``residual`` (f32 [batch, m, n] added after
         the epilogue) or ``a_dtype`` / ``b_dtype`` (the dtypes the operands
         are stored in, cast to ``in_dtype`` in a pre-pass) it calls
         bg_matmul_ex2."""
@@ -214,6 +215,7 @@ class HipRealizerBridge:
         d.out_dtype = _dtype_code(out_dtype or in_dtype, "matmul")
         d.round_f16 = 1 if round_out else 0
         d.act = int(act)
+        d.reserved = N.MATMUL_F32_UNSPLIT if f32_unsplit else 0
         out = N.handle_t()
         if residual is None and a_dtype is None and b_dtype is None:
             self._check(self._lib.bg_matmul_ex(self._ctx, C.byref(d), C.byref(out)))

@@ -261,6 +261,22 @@ struct Gemm32Shape {
   bool wide = false;  // gemm32_wide_k_kernel: 32 x 32 blocks, K split over 16 wavefronts
 };
 Gemm32Shape gemm32_shape(const bg_matmul_desc& d, bool ptrs_aligned);
+// Launch shape of the f32 GEMM on the bf16 matrix core (k_gemm_split.hip);
+// tile < 0: another kernel runs.  wide, skinny: the wide-K or the skinny kernel
+// could run; room: workspace bytes the call may take.
+struct Gemm32Split {
+  int tile = -1;
+  int slices = 1;
+  int64_t ks = 0;  // k per slice
+  int tiles_m = 0, tiles_n = 0;
+};
+Gemm32Split gemm32_split(const bg_matmul_desc& d, bool wide, bool skinny, size_t room);
+// args: the GemmArgs of the call.
+void launch_gemm32_split(bg_ctx* ctx, const Gemm32Split& g, void* args, const bg_matmul_desc& d, bool aligned,
+                         GemmWorkspace& ws);
+void plan_gemm32_split(const Gemm32Split& g, const bg_matmul_desc& d, bool aligned, bg_launch_plan& out);
+// Sums `slices` f32 partials [slices][M][N] in slice order and runs the epilogue.
+void finish_gemm_slices(bg_ctx* ctx, const void* args, int slices, const float* part);
 void plan_matmul(const bg_matmul_desc& d, bg_launch_plan& out);
 void plan_attention(const bg_attention_desc& d, bg_launch_plan& out);
 bool fa32_supported(const bg_attention_desc& d);

@@ -27,8 +27,10 @@
 //     -> store f32/f16/bf16 (the reference AMP graph CAST -> MATMUL(f16 out)
 //     -> ADD(bias, f32) in one pass).  Staging keeps every accumulator index
 //     static, so the accumulators never leave registers.
-// f32 path, gemm32_kernel: v_mfma_f32_32x32x2_f32 with k-major LDS tiles
-// (NN and NT), the same staged epilogue.
+// f32 path: k_gemm_split.hip (bf16 parts of the operands) unless the caller
+// asks for float32 matrix instructions, an operand spans 2 GiB or the output
+// is small; gemm32_kernel: v_mfma_f32_32x32x2_f32 with k-major LDS tiles (NN
+// and NT), the same staged epilogue.
 #include <algorithm>
 #include <cstdio>
 
@@ -36,173 +38,12 @@
 #include <string>
 #include <type_traits>
 
-#include "common.cuh"
 #include "core.h"
+#include "gemm_common.cuh"
 
 namespace {
 
 using namespace bgk;
-
-typedef _Float16 half8 __attribute__((ext_vector_type(8)));
-typedef __bf16 bf168 __attribute__((ext_vector_type(8)));
-typedef float float16v __attribute__((ext_vector_type(16)));
-// Native 16-byte vector (HIP's uint4 is a union-based struct, which keeps
-// arrays of it from being promoted to registers).
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-
-struct GemmArgs {
-  const void* A;
-  const void* B;
-  const float* bias;
-  void* C;
-  int64_t M, N, K;
-  int64_t lda, ldb, ldc;
-  int64_t sa, sb, sc;  // batch strides (elements)
-  int tiles_m, tiles_n;
-  int round_dtype;  // 0 none, 1 f16, 2 bf16
-  int act;          // BG_ACT_*
-  int out_dtype;    // BG_F32 / BG_F16 / BG_BF16
-  int vec_store;    // C rows can take 4-element vector stores (ldc % 4, alignment)
-  const float* R;   // residual f32 [batch][M][N] added last (NULL: none)
-  int64_t ldr, sr;  // its row and batch strides (elements)
-};
-
-// XCD-aware tile index -> (tile_m, tile_n).  Workgroups are dispatched
-// round-robin over the 8 XCDs; the tiles of one XCD are made consecutive and
-// then walked in groups of G tile-rows so neighbours share A and B panels.
-__device__ __forceinline__ void tile_coords(int pid, int tiles_m, int tiles_n, int& tm, int& tn) {
-  const int total = tiles_m * tiles_n;
-  if (total % 8 == 0) {
-    const int per = total / 8;
-    pid = (pid % 8) * per + pid / 8;
-  }
-  constexpr int G = 4;
-  const int group = pid / (G * tiles_n);
-  const int first_m = group * G;
-  const int gsz = min(G, tiles_m - first_m);
-  const int in_group = pid % (G * tiles_n);
-  tm = first_m + in_group % gsz;
-  tn = in_group / gsz;
-}
-
-__device__ __forceinline__ float epilogue_value(const GemmArgs& P, float v, float bias) {
-  if (P.round_dtype) v = round_through(v, P.round_dtype);
-  if (P.bias) v = v + bias;
-  if (P.act == BG_ACT_RELU) v = v > 0.f ? v : 0.f;
-  else if (P.act == BG_ACT_GELU_TANH) v = gelu_tanh(v);
-  return v;
-}
-
-template <int OUT>
-__device__ __forceinline__ void store_elem(char* p, float v) {
-  if constexpr (OUT == BG_F32) *reinterpret_cast<float*>(p) = v;
-  else if constexpr (OUT == BG_F16) *reinterpret_cast<uint16_t*>(p) = f32_to_f16_bits(v);
-  else *reinterpret_cast<uint16_t*>(p) = f32_to_bf16_bits(v);
-}
-
-// Epilogue in registers, stored straight to C, one 32x32 accumulator tile
-// (16 values per lane) at a time: [round to the 16-bit type] -> [+ bias[n]]
-// -> [relu] -> store, each stage behind one uniform branch per tile.
-// Scheduling fences between tiles keep the live set to one tile, so the
-// accumulators never spill.  tanh-GELU (one exponential and one reciprocal
-// per element) runs here for wavefront tiles of up to kGeluEpilogueTiles
-// accumulator tiles; wider ones leave it to a separate f32 pass over C
-// (run_matmul).
-// 32x32 MFMA accumulator layout: lane l, register e holds row
-// 8*(e/4) + 4*(l/32) + e%4, column l%32, so each store instruction writes 32
-// consecutive columns of two rows.  Addresses are a uniform per-row base plus
-// one 32-bit per-lane offset; nothing in the loop waits on memory.
-// Largest per-wavefront accumulator tile count (TM * TN) whose epilogue
-// evaluates GELU in registers.
-constexpr int kGeluEpilogueTiles = 8;
-
-template <int TM, int TN, bool FULL, int OUT>
-__device__ __forceinline__ void epilogue_tiles(const GemmArgs& P, char* C, float16v (&acc)[TM][TN],
-                                               int64_t row0, int64_t col0, const float (&bz)[TN]) {
-  constexpr int ES = OUT == BG_F32 ? 4 : 2;
-  const int lane = threadIdx.x & 63;
-  const int half = lane >> 5;
-  const int64_t cl = col0 + (lane & 31);
-  char* corner = C + (row0 * P.ldc + col0) * ES;
-  const uint32_t lane_off = uint32_t((4 * half * P.ldc + (lane & 31)) * ES);
-  const int64_t row_bytes = P.ldc * ES;
-  // Residual (f32, added after the activation): 16 values per tile, same
-  // element layout as the accumulator tile.
-  float rnext[16];
-  const float* rbase = P.R ? P.R + int64_t(blockIdx.z) * P.sr + (row0 + 4 * half) * P.ldr + cl : nullptr;
-  auto load_residual = [&](int ti, int tj) {
-    const bool ok_c = FULL || cl + tj * 32 < P.N;
-#pragma unroll
-    for (int e = 0; e < 16; ++e) {
-      const int rr = ti * 32 + 8 * (e >> 2) + (e & 3);
-      rnext[e] = (FULL || (ok_c && row0 + rr + 4 * half < P.M)) ? rbase[rr * P.ldr + tj * 32] : 0.f;
-    }
-  };
-  if (P.R) load_residual(0, 0);
-#pragma unroll
-  for (int i = 0; i < TM; ++i)
-#pragma unroll
-    for (int j = 0; j < TN; ++j) {
-      float v[16];
-#pragma unroll
-      for (int e = 0; e < 16; ++e) v[e] = acc[i][j][e];
-      if (P.round_dtype == 1) {
-#pragma unroll
-        for (int e = 0; e < 16; ++e) v[e] = round_through(v[e], 1);
-      } else if (P.round_dtype == 2) {
-#pragma unroll
-        for (int e = 0; e < 16; ++e) v[e] = round_through(v[e], 2);
-      }
-      if (P.bias) {
-#pragma unroll
-        for (int e = 0; e < 16; ++e) v[e] = v[e] + bz[j];
-      }
-      if (P.act == BG_ACT_RELU) {
-#pragma unroll
-        for (int e = 0; e < 16; ++e) v[e] = v[e] > 0.f ? v[e] : 0.f;
-      } else if constexpr (TM * TN <= kGeluEpilogueTiles) {
-        // tanh-GELU on 16 values at a time (the tile fence below keeps the
-        // compiler from interleaving tiles); wider wavefront tiles leave no
-        // registers for it and take the separate f32 pass instead.
-        if (P.act == BG_ACT_GELU_TANH) {
-#pragma unroll
-          for (int e = 0; e < 16; ++e) v[e] = gelu_tanh(v[e]);
-        }
-      }
-      const bool col_ok = FULL || cl + j * 32 < P.N;
-      if (P.R) {
-        // The residual of this tile was loaded one tile ahead (before the
-        // previous tile's stores), so its wait does not queue behind them.
-        float cur[16];
-#pragma unroll
-        for (int e = 0; e < 16; ++e) cur[e] = rnext[e];
-        if (i * TN + j + 1 < TM * TN) load_residual((i * TN + j + 1) / TN, (i * TN + j + 1) % TN);
-#pragma unroll
-        for (int e = 0; e < 16; ++e) v[e] = v[e] + cur[e];
-      }
-#pragma unroll
-      for (int e = 0; e < 16; ++e) {
-        const int rr = i * 32 + 8 * (e >> 2) + (e & 3);
-        if (FULL || (col_ok && row0 + rr + 4 * half < P.M))
-          store_elem<OUT>(corner + rr * row_bytes + lane_off + j * 32 * ES, v[e]);
-      }
-      __builtin_amdgcn_sched_barrier(0);
-    }
-}
-
-template <int TM, int TN, bool FULL>
-__device__ __forceinline__ void direct_epilogue(const GemmArgs& P, char* C, float16v (&acc)[TM][TN],
-                                                int64_t row0, int64_t col0) {
-  const int lane = threadIdx.x & 63;
-  const int64_t cl = col0 + (lane & 31);
-  float bz[TN];
-#pragma unroll
-  for (int j = 0; j < TN; ++j)
-    bz[j] = (P.bias && (FULL || cl + j * 32 < P.N)) ? P.bias[cl + j * 32] : 0.f;
-  if (P.out_dtype == BG_F32) epilogue_tiles<TM, TN, FULL, BG_F32>(P, C, acc, row0, col0, bz);
-  else if (P.out_dtype == BG_F16) epilogue_tiles<TM, TN, FULL, BG_F16>(P, C, acc, row0, col0, bz);
-  else epilogue_tiles<TM, TN, FULL, BG_BF16>(P, C, acc, row0, col0, bz);
-}
 
 // ---- 16-bit MFMA kernel ---------------------------------------------------------
 
@@ -1076,12 +917,17 @@ namespace bg {
 // step, so such GEMMs take the wide-K kernel instead (32 x 32 blocks, K
 // split over the wavefronts of a workgroup and summed through LDS, one
 // launch).
+// Rows of A and B (along K, or along N for a [K][N] B) allow 16-byte loads.
+static bool gemm32_rows_aligned(const bg_matmul_desc& d, bool ptrs_aligned) {
+  return ptrs_aligned && d.lda % 4 == 0 && d.ldb % 4 == 0 && d.k % 4 == 0 && (d.trans_b || d.n % 4 == 0) &&
+         d.stride_a % 4 == 0 && d.stride_b % 4 == 0;
+}
+
 Gemm32Shape gemm32_shape(const bg_matmul_desc& d, bool ptrs_aligned) {
   Gemm32Shape g;
   g.tiles_m = int((d.m + 127) / 128);
   g.tiles_n = int((d.n + 127) / 128);
-  g.aligned = ptrs_aligned && d.lda % 4 == 0 && d.ldb % 4 == 0 && d.k % 4 == 0 && (d.trans_b || d.n % 4 == 0) &&
-              d.stride_a % 4 == 0 && d.stride_b % 4 == 0;
+  g.aligned = gemm32_rows_aligned(d, ptrs_aligned);
   const int64_t nk = (d.k + BK32 - 1) / BK32;
   const int64_t tiles = int64_t(g.tiles_m) * g.tiles_n;
   if (d.batch == 1 && tiles <= 16 && nk >= 8) {
@@ -1114,8 +960,8 @@ static bool gelu_in_epilogue(const bg_matmul_desc& d, const char* a, const char*
 
 // a / b point at the operands' storage (d.offset_a / d.offset_b are applied
 // here); bias is f32 [N] or NULL.
-// Skinny GEMMs: at most 512 rows for f32 (blocks of 64) or 64 for 16-bit,
-// a K of 512+, fewer 128-column tiles than CUs and one batch (the tiled
+// Skinny GEMMs: at most 512 rows for f32 (blocks of 64; above 32 rows only
+// where the product is not split) or 64 for 16-bit, a K of 512+, fewer 128-column tiles than CUs and one batch (the tiled
 // kernels would leave most of the chip idle).
 // K slices of at least 256 (and multiples of 64: four wavefronts interleave
 // the steps) until about 256 workgroups stream B; a workspace with less
@@ -1124,6 +970,10 @@ struct SkinnyPlan {
   bool on = false;
   int64_t ntiles = 0, rblocks = 1, nsplit = 1, ks = 0;
 };
+
+static size_t workspace_room(const GemmWorkspace& ws) {
+  return ws.fixed ? ws.cap - std::min(ws.cap, ws.used) : SIZE_MAX;
+}
 
 static SkinnyPlan skinny_plan(const bg_matmul_desc& d, int dt, size_t room) {
   SkinnyPlan sp;
@@ -1150,10 +1000,16 @@ static SkinnyPlan skinny_plan(const bg_matmul_desc& d, int dt, size_t room) {
   return sp;
 }
 
+void finish_gemm_slices(bg_ctx* ctx, const void* args, int slices, const float* part) {
+  const GemmArgs& P = *static_cast<const GemmArgs*>(args);
+  bg::dispatch(ctx, gemm_skinny_finish_kernel, dim3(static_cast<unsigned>((P.M * P.N + 255) / 256)), dim3(256), 0, P,
+               slices, part);
+}
+
 // Operands must allow 16-byte loads along K (the caller checks); tb: B is
 // [N][K].  Returns false when the problem is not skinny.
 static bool launch_skinny(bg_ctx* ctx, const bg_matmul_desc& d, GemmArgs& P, GemmWorkspace& ws, int dt, bool tb) {
-  const SkinnyPlan sp = skinny_plan(d, dt, ws.fixed ? ws.cap - std::min(ws.cap, ws.used) : SIZE_MAX);
+  const SkinnyPlan sp = skinny_plan(d, dt, workspace_room(ws));
   if (!sp.on) return false;
   const int64_t nsplit = sp.nsplit, ks = sp.ks;
   float* part = nsplit > 1 ? static_cast<float*>(ws.get(size_t(nsplit * d.m * d.n) * 4, 3)) : nullptr;
@@ -1176,9 +1032,7 @@ static bool launch_skinny(bg_ctx* ctx, const bg_matmul_desc& d, GemmArgs& P, Gem
   if (dt == BG_F32) by_mt(std::integral_constant<int, BG_F32>{});
   else if (dt == BG_F16) by_mt(std::integral_constant<int, BG_F16>{});
   else by_mt(std::integral_constant<int, BG_BF16>{});
-  if (nsplit > 1)
-    bg::dispatch(ctx, gemm_skinny_finish_kernel, dim3(static_cast<unsigned>((d.m * d.n + 255) / 256)), dim3(256), 0,
-                 P, ns, static_cast<const float*>(part));
+  if (nsplit > 1) finish_gemm_slices(ctx, &P, ns, part);
   return true;
 }
 
@@ -1220,6 +1074,12 @@ static void run_gemm(bg_ctx* ctx, const bg_matmul_desc& d, const char* a, const 
     P.tiles_n = g.tiles_n;
     const bool aligned = g.aligned;
     Profile prof(ctx, "gemm_f32", bytes, flops);
+    const size_t room = workspace_room(ws);
+    const Gemm32Split gs = gemm32_split(d, g.wide, aligned && skinny_plan(d, BG_F32, room).on, room);
+    if (gs.tile >= 0) {
+      launch_gemm32_split(ctx, gs, &P, d, gemm32_rows_aligned(d, aligned_to(P.A, 16) && aligned_to(P.B, 16)), ws);
+      return;
+    }
     if (g.wide) {
       const dim3 grid(unsigned(g.tiles_m * g.tiles_n));
       const dim3 block(kWideWaves * 64);
@@ -1408,6 +1268,21 @@ void plan_matmul(const bg_matmul_desc& d0, bg_launch_plan& out) {
   out.k_slices = 1;
   out.n_launches = 1;
   bg_launch_plan_entry& e = out.launch[0];
+  auto finish = [&] {
+    out.n_launches = 2;
+    bg_launch_plan_entry& f = out.launch[1];
+    std::snprintf(f.family, sizeof f.family, "%s", "gemm_skinny_finish_kernel");
+    f.n_targs = 0;
+    f.grid[0] = (d.m * d.n + 255) / 256; f.grid[1] = 1; f.grid[2] = 1;
+    f.block[0] = 256; f.block[1] = 1; f.block[2] = 1;
+  };
+  const SkinnyPlan sp = g.aligned ? skinny_plan(d, BG_F32, SIZE_MAX) : SkinnyPlan{};
+  const Gemm32Split gs = gemm32_split(d, g.wide, sp.on, SIZE_MAX);
+  if (gs.tile >= 0) {
+    plan_gemm32_split(gs, d, gemm32_rows_aligned(d, ptrs), out);
+    if (gs.slices > 1) finish();
+    return;
+  }
   if (g.wide) {
     out.tile_m = 32;
     out.tile_n = 32;
@@ -1423,7 +1298,6 @@ void plan_matmul(const bg_matmul_desc& d0, bg_launch_plan& out) {
     e.block[0] = kWideWaves * 64; e.block[1] = 1; e.block[2] = 1;
     return;
   }
-  const SkinnyPlan sp = g.aligned ? skinny_plan(d, BG_F32, SIZE_MAX) : SkinnyPlan{};
   if (sp.on) {
     const int mt = d.m <= 32 ? 1 : 2;
     out.tile_m = 32 * mt;
@@ -1439,14 +1313,7 @@ void plan_matmul(const bg_matmul_desc& d0, bg_launch_plan& out) {
     e.targs[2] = d.trans_b ? 1 : 0;
     e.grid[0] = sp.ntiles * sp.nsplit; e.grid[1] = sp.rblocks; e.grid[2] = 1;
     e.block[0] = 1024; e.block[1] = 1; e.block[2] = 1;
-    if (sp.nsplit > 1) {
-      out.n_launches = 2;
-      bg_launch_plan_entry& f = out.launch[1];
-      std::snprintf(f.family, sizeof f.family, "%s", "gemm_skinny_finish_kernel");
-      f.n_targs = 0;
-      f.grid[0] = (d.m * d.n + 255) / 256; f.grid[1] = 1; f.grid[2] = 1;
-      f.block[0] = 256; f.block[1] = 1; f.block[2] = 1;
-    }
+    if (sp.nsplit > 1) finish();
     return;
   }
   out.tile_m = 128;

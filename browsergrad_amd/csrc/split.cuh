@@ -1,0 +1,48 @@
+// float32 products on the bf16 matrix core: every float32 value is the exact
+// sum of three bf16 values, x = x1 + x2 + x3 (round to nearest at each step:
+// 24 significand bits as 8 + 8 + 8 with signed remainders), and a product is
+// taken as x1 y1 + x1 y2 + x2 y1 + x2 y2 + x1 y3 + x3 y1.  What is dropped,
+// x2 y3 + x3 y2 + x3 y3, is below 2^-26 |x y|, a quarter of the rounding of a
+// float32 product; sums stay in float32 accumulators.
+#pragma once
+
+#include "common.cuh"
+
+namespace bgk {
+
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef uint32_t u32x4s __attribute__((ext_vector_type(4)));
+
+// Smallest magnitude that splits exactly: the third part of x reaches down to
+// 2^-23 |x|, and bf16's smallest step is 2^-133.  split8 keeps the minimum of
+// 2 * magnitude bits - 2 over the nonzero values it sees (zero wraps to the
+// top); a kernel whose minimum is below kSplitMin redoes its tile in float32.
+constexpr uint32_t kSplitTop = 0xffffffffu;
+constexpr uint32_t kSplitMin = ((127u - 109u) << 24) - 2u;  // 2^-109
+
+// Splits two values into the packed bf16 parts.
+__device__ __forceinline__ void split2(float x0, float x1, uint32_t& p1, uint32_t& p2, uint32_t& p3, uint32_t& low) {
+  const f32x2 v = {x0, x1};
+  low = min(low, min((__float_as_uint(x0) << 1) - 2u, (__float_as_uint(x1) << 1) - 2u));
+  p1 = __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2));
+  const f32x2 r = {x0 - __uint_as_float(p1 << 16), x1 - __uint_as_float(p1 & 0xffff0000u)};
+  p2 = __builtin_bit_cast(uint32_t, __builtin_convertvector(r, bf16x2));
+  const f32x2 q = {r[0] - __uint_as_float(p2 << 16), r[1] - __uint_as_float(p2 & 0xffff0000u)};
+  p3 = __builtin_bit_cast(uint32_t, __builtin_convertvector(q, bf16x2));
+}
+
+// Splits eight consecutive values.
+__device__ __forceinline__ void split8(const float (&x)[8], u32x4s& p1, u32x4s& p2, u32x4s& p3, uint32_t& low) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    uint32_t a, b, c;
+    split2(x[2 * i], x[2 * i + 1], a, b, c, low);
+    p1[i] = a;
+    p2[i] = b;
+    p3[i] = c;
+  }
+}
+
+}  // namespace bgk

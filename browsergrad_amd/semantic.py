@@ -389,6 +389,8 @@ def prepare_semantic_gemm(m: int, n: int, k: int, *, max_transient_working_set_b
     d.batch, d.m, d.n, d.k = 1, m, n, k
     d.lda, d.ldb, d.ldc = k, n, n
     d.trans_b, d.in_dtype, d.out_dtype = 0, N.BG_F32, N.BG_F32
+    # The certificate's overflow proof needs monotone partial sums.
+    d.reserved = N.MATMUL_F32_UNSPLIT
     plan = launch_plan("gemm", d)
     lds = _workgroup_limits(plan, max_workgroup_invocations, max_workgroup_storage_bytes, code)
     main = plan["launches"][0]
@@ -602,7 +604,8 @@ def run_semantic_gemm(bridge: Any, prepared: PreparedSemanticGemm, certificate: 
     try:
         dl.check()
         hc, launches = _run_logged(
-            bridge, lambda: bridge.matmul_ex(ha, hb, m=m, n=n, k=k, in_dtype="float32", out_dtype="float32"))
+            bridge, lambda: bridge.matmul_ex(ha, hb, m=m, n=n, k=k, in_dtype="float32", out_dtype="float32",
+                                             f32_unsplit=True))
         try:
             check_launches(prepared.plan, launches, "BG-WEBGPU-GEMM-VALIDATION")
             check_layout(prepared.layout, {"lhs": bridge.handle_info(ha), "rhs": bridge.handle_info(hb),

@@ -171,8 +171,16 @@ typedef struct bg_matmul_desc {
   int32_t out_dtype;     /* BG_F32 / BG_F16 / BG_BF16 */
   int32_t round_f16;     /* round accumulator to the intermediate dtype before bias */
   int32_t act;           /* BG_ACT_* */
-  int32_t reserved;
+  int32_t reserved;      /* 0, or BG_MATMUL_F32_UNSPLIT */
 } bg_matmul_desc;
+
+/* An f32 product is taken from three bf16 parts of each operand (every f32
+ * is their exact sum) on the bf16 matrix core, six partial products each,
+ * with f32 sums: at least as close to the exact result as float32 products,
+ * but the parts are signed, so sums of non-negative terms need not be
+ * monotone.  With this value in `reserved` every product is formed by a
+ * float32 matrix instruction (proofs that rest on monotone partial sums). */
+#define BG_MATMUL_F32_UNSPLIT 1
 
 /* Extras for bg_matmul_ex2.  The epilogue is
  *   y = act([round](acc) + bias) + residual
