@@ -43,6 +43,7 @@ OPS = {
 RED_NONE, RED_SUM, RED_MAX, RED_MEAN, RED_MIN = range(5)
 ACT_NONE, ACT_RELU, ACT_GELU_TANH = range(3)
 MATMUL_F32_UNSPLIT = 1
+ATTENTION_TILED = 1
 
 handle_t = C.c_uint64
 

@@ -287,9 +287,10 @@ class HipRealizerBridge:
                      q_view: Tuple[int, int, int, int] = (0, 0, 0, 0),
                      k_view: Tuple[int, int, int, int] = (0, 0, 0, 0),
                      v_view: Tuple[int, int, int, int] = (0, 0, 0, 0),
-                     o_strides: Tuple[int, int, int] = (0, 0, 0)) -> int:
+                     o_strides: Tuple[int, int, int] = (0, 0, 0), tiled: bool = False) -> int:
         """q/k/v_view = (offset, batch stride, head stride, seq stride); zeros
-        mean contiguous [B, H, S, D]."""
+        mean contiguous [B, H, S, D].  ``tiled``: the tiled kernels also for
+        a few query rows (BG_ATTENTION_TILED)."""
         a = N.AttentionDesc()
         a.q, a.k, a.v = int(q), int(k), int(v)
         a.batch, a.heads, a.sq, a.sk, a.d = int(batch), int(heads), int(sq), int(sk), int(d)
@@ -302,6 +303,7 @@ class HipRealizerBridge:
         a.in_dtype = _dtype_code(in_dtype, "flash_attention")
         a.out_dtype = _dtype_code(out_dtype or in_dtype, "flash_attention")
         a.round_scores = 1 if round_scores else 0
+        a.reserved = N.ATTENTION_TILED if tiled else 0
         out = N.handle_t()
         self._check(self._lib.bg_attention_ex(self._ctx, C.byref(a), C.byref(out)))
         return int(out.value)

@@ -279,6 +279,11 @@ void plan_gemm32_split(const Gemm32Split& g, const bg_matmul_desc& d, bool align
 void finish_gemm_slices(bg_ctx* ctx, const void* args, int slices, const float* part);
 void plan_matmul(const bg_matmul_desc& d, bg_launch_plan& out);
 void plan_attention(const bg_attention_desc& d, bg_launch_plan& out);
+// Attention of at most four query rows (k_attn_decode.hip): key slices of the
+// call, 0 where another kernel takes it; launch returns false then.
+int attention_decode_slices(const bg_attention_desc& d, bool ptrs_aligned);
+bool launch_attention_decode(bg_ctx* ctx, const bg_attention_desc& d, const char* q, const char* k, const char* v,
+                             void* o);
 bool fa32_supported(const bg_attention_desc& d);
 void launch_fa32(bg_ctx* ctx, const bg_attention_desc& d, const float* q, const float* k, const float* v,
                  const float* mask, int64_t m_sb, int64_t m_sh, int64_t m_ss, void* o);

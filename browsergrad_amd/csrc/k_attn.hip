@@ -1830,6 +1830,11 @@ void launch_attention(bg_ctx* ctx, const bg_attention_desc& d, const Record& q, 
                        d.v_sb % 4 == 0 && d.v_sh % 4 == 0 && d.o_sb % 4 == 0 && d.o_sh % 4 == 0 &&
                        al(qp, 16) && al(kp, 16) && al(vp, 8) && al(out.ptr(), 16) &&
                        d.batch * d.heads <= 0x7fffffff && sq <= (1 << 30) && sk <= (1 << 30);
+  {
+    Profile prof(ctx, d.in_dtype == BG_F32 ? "attention_f32" : d.in_dtype == BG_F16 ? "attention_f16" : "attention_bf16",
+                 bytes, flops);
+    if (launch_attention_decode(ctx, d, qp, kp, vp, out.ptr())) return;
+  }
   if (d.in_dtype == BG_F32 && fa32_supported(d)) {
     Profile prof(ctx, "attention_f32", bytes, flops);
     launch_fa32(ctx, d, reinterpret_cast<const float*>(qp), reinterpret_cast<const float*>(kp),

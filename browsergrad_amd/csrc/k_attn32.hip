@@ -351,6 +351,28 @@ void plan_attention(const bg_attention_desc& d0, bg_launch_plan& out) {
   const bool ptrs = (d.q_off % 4) == 0 && (d.k_off % 4) == 0 && (d.v_off % 4) == 0;
   const int dp = d.d <= 16 ? 16 : d.d <= 32 ? 32 : 64;
   out = bg_launch_plan{};
+  if (const int slices = attention_decode_slices(d, ptrs)) {
+    const int nq = d.sq == 1 ? 1 : d.sq == 2 ? 2 : 4;
+    out.tile_m = nq;
+    out.tile_n = 1;
+    out.tile_k = int32_t(d.d);
+    out.k_slices = slices;
+    out.lds_bytes = 16 * nq * 66 * 4;
+    out.workspace_bytes = slices > 1 ? d.batch * d.heads * slices * d.sq * (d.d + 2) * 4 : 0;
+    out.n_launches = slices > 1 ? 2 : 1;
+    auto entry = [&](int i, const char* family, int a0, int a1, int64_t gx, int64_t gy, int threads) {
+      bg_launch_plan_entry& e = out.launch[i];
+      std::snprintf(e.family, sizeof e.family, "%s", family);
+      e.n_targs = a1 ? 2 : 1;
+      e.targs[0] = a0;
+      e.targs[1] = a1;
+      e.grid[0] = gx; e.grid[1] = gy; e.grid[2] = 1;
+      e.block[0] = threads; e.block[1] = 1; e.block[2] = 1;
+    };
+    entry(0, "attention_decode_kernel", BG_F32, nq, d.batch * d.heads, slices, 1024);
+    if (slices > 1) entry(1, "attention_decode_merge_kernel", BG_F32, 0, d.batch * d.heads * d.sq, 1, 64);
+    return;
+  }
   out.tile_m = kBQ;
   out.tile_n = kBK;
   out.tile_k = dp;

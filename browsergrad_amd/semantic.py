@@ -481,6 +481,7 @@ def prepare_semantic_attention(batch: int, heads: int, q_len: int, k_len: int, h
     d.batch, d.heads, d.sq, d.sk, d.d = batch, heads, q_len, k_len, head_dim
     d.scale, d.causal = sc, 1 if causal else 0
     d.in_dtype = d.out_dtype = N.BG_F32
+    d.reserved = N.ATTENTION_TILED  # the artifacts describe the tiled kernel
     plan = launch_plan("attention", d)
     lds = _workgroup_limits(plan, max_workgroup_invocations, max_workgroup_storage_bytes, code)
     main = plan["launches"][0]
@@ -705,7 +706,7 @@ def run_semantic_attention(bridge: Any, prepared: PreparedSemanticAttention, que
         dl.check()
         ho, launches = _run_logged(bridge, lambda: bridge.attention_ex(
             hs[0], hs[1], hs[2], batch=batch, heads=heads, sq=q_len, sk=k_len, d=head_dim, scale=prepared.scale,
-            causal=prepared.causal, in_dtype="float32", out_dtype="float32"))
+            causal=prepared.causal, in_dtype="float32", out_dtype="float32", tiled=True))
         try:
             check_launches(prepared.plan, launches, "BG-WEBGPU-ATTENTION-VALIDATION")
             check_layout(prepared.layout, {"query": bridge.handle_info(hs[0]), "key": bridge.handle_info(hs[1]),

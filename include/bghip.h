@@ -227,8 +227,12 @@ typedef struct bg_attention_desc {
   int32_t in_dtype;     /* BG_F16 / BG_BF16 (MFMA) or BG_F32 */
   int32_t out_dtype;
   int32_t round_scores;
-  int32_t reserved;
+  int32_t reserved;     /* 0, or BG_ATTENTION_TILED */
 } bg_attention_desc;
+
+/* In `reserved`: calls of a few query rows, which by default stream K
+ * and V without matrix instructions, run the tiled kernels as well. */
+#define BG_ATTENTION_TILED 1
 
 /* Resource snapshot (realizer.ts:287-298 WebGpuResourceSnapshot). */
 typedef struct bg_snapshot {
