@@ -290,7 +290,8 @@ class HipRealizerBridge:
                      o_strides: Tuple[int, int, int] = (0, 0, 0), tiled: bool = False) -> int:
         """q/k/v_view = (offset, batch stride, head stride, seq stride); zeros
         mean contiguous [B, H, S, D].  ``tiled``: the tiled kernels also for
-        a few query rows (BG_ATTENTION_TILED)."""
+        a few query rows, and float32 products by float32 matrix instructions
+        (BG_ATTENTION_TILED)."""
         a = N.AttentionDesc()
         a.q, a.k, a.v = int(q), int(k), int(v)
         a.batch, a.heads, a.sq, a.sk, a.d = int(batch), int(heads), int(sq), int(sk), int(d)

@@ -47,6 +47,7 @@
 
 #include "common.cuh"
 #include "core.h"
+#include "split.cuh"
 
 namespace {
 
@@ -277,8 +278,360 @@ __global__ void __launch_bounds__(kNW * 64, 2) fa32_fwd_kernel(Fa32Args P) {
     }
 }
 
-}  // namespace
+// ---- the same attention on the bf16 matrix core ------------------------------------
+//
+// split_fa32_fwd_kernel keeps the tiles and the numerics above and forms its
+// products from three bf16 parts of Q, K, V and P (split.cuh): 24
+// v_mfma_f32_32x32x16_bf16 of 32 cycles where float32 takes 32 MFMAs of 64.
+//   * 512 threads: wavefront w takes queries 32 (w % 4) .. +31 and the 32-key
+//     half w / 4 of every tile, with its own maximum, sum and output; the
+//     halves merge through LDS at the end.  Four more wavefronts share the
+//     cost of splitting a tile and halve the chain of a tile's products.
+//   * K and V are split once per workgroup on the way to LDS, V transposed:
+//     eight keys of one column per 16-byte unit, in the key order of a lane's
+//     accumulator registers, so P again never leaves the registers.  Two
+//     buffers; the split of tile t + 1 runs beside the score MFMAs of tile t
+//     (seven vector instructions an MFMA), tile t + 2 loads meanwhile.
+// Bound: neither pipe alone: per tile a SIMD's two wavefronts need about 3100
+// cycles of the matrix core and 3000 of the vector unit (exponentials, the
+// splits of P), which overlap only in the scores.  B4 H12 S1000 D64 causal 107
+// -> 60 us, B8 H16 S2048 causal 614 -> 462, one head of 2048 163 -> 92 (a
+// one-buffer form of four wavefronts, two workgroups a CU: 99 / 458 / 152).
+// Error against float64, 2-norm, B4 H12 S1000: 2.2e-7 (fa32_fwd_kernel 3.3e-7).
+// The parts hold values down to 2^-109 and finite ones; a workgroup that saw
+// others, or whose sums are not finite, redoes its queries one at a time in
+// float32 (fa32_plain).  Weights P below 2^-109 of their row's largest lose
+// bits: an error under 2^-133 max |v|.
 
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+constexpr int kSplitNT = 512;  // wavefront w: queries 32 (w % 4) .., keys 32 (w / 4) .. of every tile
+
+// Queries q0w .. +31 of one wavefront in float32: one key per lane for the
+// scores, one output column per lane for P V.
+__device__ __forceinline__ void fa32_plain(const Fa32Args& P, const float* Qp, const float* Kp,
+                                                     const float* Vp, const float* Mp, int64_t ohead, int q0w) {
+  const int lane = threadIdx.x & 63;
+  const bool col = lane < P.D;
+  for (int qi = q0w; qi < min(q0w + kQW, P.Sq); ++qi) {
+    const int keys = P.causal ? min(P.Sk, qi + 1) : P.Sk;
+    const float* qr = Qp + int64_t(qi) * P.q_ss;
+    float m = kMSentinel, l = 0.f, o = 0.f;
+    for (int j0 = 0; j0 < keys; j0 += 64) {
+      const int j = j0 + lane;
+      float s = -INFINITY;
+      if (j < keys) {
+        s = 0.f;
+        for (int d = 0; d < P.D; ++d) s = __builtin_fmaf(qr[d] * P.sl2, Kp[int64_t(j) * P.k_ss + d], s);
+        if (Mp) s = __builtin_fmaf(Mp[int64_t(qi) * P.m_ss + j], kLog2e, s);
+      }
+      float mt = s;
+      for (int x = 1; x < 64; x <<= 1) mt = fmaxf(mt, __shfl_xor(mt, x));
+      const float m_new = fmaxf(m, mt), alpha = __builtin_amdgcn_exp2f(m - m_new);
+      m = m_new;
+      const float p = __builtin_amdgcn_exp2f(s - m_new);
+      l = l * alpha + bgk::wave_sum(p);
+      o *= alpha;
+      for (int x = 0; x < min(64, keys - j0); ++x) {
+        const float px = __shfl(p, x);
+        if (col) o = __builtin_fmaf(px, Vp[int64_t(j0 + x) * P.v_ss + lane], o);
+      }
+    }
+    if (col)
+      bgk::store_from_f32(P.o, P.out_dtype, ohead + int64_t(qi) * P.o_ss + lane, l > 0.f ? o * (1.0f / l) : l == l ? 0.f : l);
+  }
+}
+
+template <int DP, bool VEC>
+__global__ void __launch_bounds__(kSplitNT, 2) split_fa32_fwd_kernel(Fa32Args P, uint32_t k_bytes,
+                                                                     uint32_t v_bytes) {
+  constexpr int NC = DP / 16;            // 16-deep d steps of the scores
+  constexpr int NDB = DP > 32 ? 2 : 1;   // 32-row blocks of O^T
+  constexpr int KU = 2 * NC * 64;        // 16-byte units per plane: 64 keys x DP / 8 chunks
+  constexpr int VU = 4 * NDB * 64;       // 32 NDB columns x 8 sets of eight keys
+  constexpr int NK = (KU + kSplitNT - 1) / kSplitNT, NV = (VU + kSplitNT - 1) / kSplitNT;
+  constexpr int BUF = 3 * (KU + VU);
+  __shared__ u32x4 smem[2 * BUF > 4 * 64 * 9 ? 2 * BUF : 4 * 64 * 9];
+
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int hi = lane >> 5, l32 = lane & 31;
+  const int bh = blockIdx.x;
+  const int qblk = P.n_qblocks - 1 - int(blockIdx.y);  // heavy (late) blocks first
+  const int b = bh / P.H, h = bh % P.H;
+  const int q0 = qblk * kBQ, q0w = q0 + (w & 3) * kQW, qi = q0w + l32;
+  const int hh = w >> 2;
+  const float* Qp = P.q + b * P.q_sb + h * P.q_sh;
+  const float* Kp = P.k + b * P.k_sb + h * P.k_sh;
+  const float* Vp = P.v + b * P.v_sb + h * P.v_sh;
+  const float* Mp = P.mask ? P.mask + b * P.m_sb + h * P.m_sh : nullptr;
+  const int nt_all = (P.Sk + kBK - 1) / kBK;
+  const int nt = P.causal ? min(nt_all, (q0 + kBQ + kBK - 1) / kBK) : nt_all;
+  uint32_t low = bgk::kSplitTop;
+
+  // B operand of the scores: Q[qi][16 c + 8 hi + j] * scale * log2(e).
+  bgk::bf16x8 qf[NC][3];
+#pragma unroll
+  for (int c = 0; c < NC; ++c) {
+    float x[8];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const float4v v = load4<VEC>(Qp, P.q_ss, qi, P.Sq, 4 * c + 2 * hi + i, P.D);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) x[4 * i + j] = v[j] * P.sl2;
+    }
+    u32x4 p1, p2, p3;
+    bgk::split8(x, p1, p2, p3, low);
+    qf[c][0] = __builtin_bit_cast(bgk::bf16x8, p1);
+    qf[c][1] = __builtin_bit_cast(bgk::bf16x8, p2);
+    qf[c][2] = __builtin_bit_cast(bgk::bf16x8, p3);
+  }
+
+  // Staging: K unit (key, 8-deep chunk), V unit (column, set of eight keys:
+  // set 2 g + x holds keys 16 g + 4 x + {0..3, 8..11}).  Buffer loads: rows
+  // past Sk and columns past D take an offset beyond the head's span and read 0.
+  const __amdgpu_buffer_rsrc_t rk = __builtin_amdgcn_make_buffer_rsrc((void*)Kp, (short)0, int(k_bytes), 0x00020000);
+  const __amdgpu_buffer_rsrc_t rv = __builtin_amdgcn_make_buffer_rsrc((void*)Vp, (short)0, int(v_bytes), 0x00020000);
+  // (An offset of the high bit is beyond any span; it is or-ed in, which keeps
+  // the loads free of branches.  Tiles past the last one read nothing but 0.)
+  const uint32_t k_row = uint32_t(P.k_ss) * 4, v_row = uint32_t(P.v_ss) * 4;
+  auto oob = [](bool ok) { return ok ? 0u : 0x80000000u; };
+  uint32_t k_at[NK], k_out[NK][VEC ? 2 : 8], v_at[NV], v_out[NV];
+#pragma unroll
+  for (int s = 0; s < NK; ++s) {
+    const int u = tid + s * kSplitNT, c = 8 * (u % (2 * NC));
+    k_at[s] = uint32_t(u / (2 * NC)) * k_row + c * 4;
+#pragma unroll
+    for (int i = 0; i < (VEC ? 2 : 8); ++i) k_out[s][i] = oob((KU % kSplitNT == 0 || u < KU) && c + (VEC ? 4 : 1) * i < P.D);
+  }
+#pragma unroll
+  for (int s = 0; s < NV; ++s) {
+    const int u = tid + s * kSplitNT, d = u % (32 * NDB), set = u / (32 * NDB);
+    v_at[s] = uint32_t(16 * (set >> 1) + 4 * (set & 1)) * v_row + d * 4;
+    v_out[s] = oob((VU % kSplitNT == 0 || u < VU) && d < P.D);
+  }
+  float kx[NK][8], vx[NV][8];
+  auto fetch = [&](int t) {
+    const int left = P.Sk - t * kBK;  // rows of the tile that exist
+    const uint32_t k_tile = left > 0 ? uint32_t(t * kBK) * k_row : 0u, v_tile = left > 0 ? uint32_t(t * kBK) * v_row : 0u;
+#pragma unroll
+    for (int s = 0; s < NK; ++s) {
+      const uint32_t off = k_at[s] + k_tile, row = oob((tid + s * kSplitNT) / (2 * NC) < left);
+      if constexpr (VEC) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(rk, (off + 16 * i) | row | k_out[s][i], 0, 0);
+#pragma unroll
+          for (int j = 0; j < 4; ++j) kx[s][4 * i + j] = __uint_as_float(v[j]);
+        }
+      } else {
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+          kx[s][j] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rk, (off + 4 * j) | row | k_out[s][j], 0, 0));
+      }
+    }
+#pragma unroll
+    for (int s = 0; s < NV; ++s) {
+      const int set = (tid + s * kSplitNT) / (32 * NDB), key0 = 16 * (set >> 1) + 4 * (set & 1);
+      const uint32_t off = v_at[s] + v_tile;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const int kj = (j & 3) + 8 * (j >> 2);
+        vx[s][j] = __uint_as_float(
+            __builtin_amdgcn_raw_buffer_load_b32(rv, (off + kj * v_row) | v_out[s] | oob(key0 + kj < left), 0, 0));
+      }
+    }
+  };
+  auto put = [&](u32x4* st, int plane, const float (&x)[8]) {
+    u32x4 p1, p2, p3;
+    bgk::split8(x, p1, p2, p3, low);
+    st[0] = p1;
+    st[plane] = p2;
+    st[2 * plane] = p3;
+  };
+  auto stash = [&](int buf) {
+    u32x4* st = smem + buf * BUF;
+#pragma unroll
+    for (int s = 0; s < NK; ++s) {
+      const int u = tid + s * kSplitNT, key = u / (2 * NC), c = u % (2 * NC);
+      if (KU % kSplitNT == 0 || u < KU)
+        put(st + ((key >> 5) * NC + (c >> 1)) * 64 + (c & 1) * 32 + ((key & 31) ^ ((c & 1) * 8)), KU, kx[s]);
+    }
+#pragma unroll
+    for (int s = 0; s < NV; ++s) {
+      const int u = tid + s * kSplitNT, d = u % (32 * NDB), set = u / (32 * NDB);
+      if (VU % kSplitNT == 0 || u < VU)
+        put(st + 3 * KU + ((set >> 1) * NDB + (d >> 5)) * 64 + (set & 1) * 32 + ((d & 31) ^ ((set & 1) * 8)), VU,
+            vx[s]);
+    }
+  };
+  // Parts (i, j) of the six products, small ones first.
+  constexpr int QA[6] = {2, 0, 1, 1, 0, 0}, QB[6] = {0, 2, 1, 0, 1, 0};
+  const int lu = lane ^ (hi << 3);
+
+  float16v acc[NDB];
+#pragma unroll
+  for (int db = 0; db < NDB; ++db)
+#pragma unroll
+    for (int e = 0; e < 16; ++e) acc[db][e] = 0.f;
+  float m_run = kMSentinel, l_run = 0.f;
+  float16v s;
+  float mv[16];  // mask of the half, loaded ahead of the products (row and key clamped)
+  // Scores of tile t, and beside their MFMAs the split of tile t + 1 from the
+  // loaded registers into the other buffer.  (A half that the causal mask hides
+  // computes scores that are not used.)
+  auto scores = [&](int t) {
+    if (Mp) {
+      const float* mrow = Mp + int64_t(min(qi, P.Sq - 1)) * P.m_ss;
+#pragma unroll
+      for (int e = 0; e < 16; ++e) mv[e] = mrow[min(t * kBK + hh * 32 + 8 * (e >> 2) + 4 * hi + (e & 3), P.Sk - 1)];
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    const u32x4* ks = smem + (t & 1) * BUF + hh * NC * 64 + lu;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) s[e] = 0.f;
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+      bgk::bf16x8 kf[3];
+#pragma unroll
+      for (int p = 0; p < 3; ++p) kf[p] = __builtin_bit_cast(bgk::bf16x8, ks[p * KU + c * 64]);
+#pragma unroll
+      for (int p = 0; p < 6; ++p)
+        s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[QA[p]], qf[c][QB[p]], s, 0, 0, 0);
+    }
+    stash((t + 1) & 1);
+    __builtin_amdgcn_sched_group_barrier(0x100, 3, 0);
+#pragma unroll
+    for (int q = 0; q < 6 * NC; ++q) {
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(0x002, 7, 0);
+      if (q % 6 == 1) __builtin_amdgcn_sched_group_barrier(0x100, 3, 0);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  // Step t loads tile t + 2, takes tile t's softmax and P V, and after the
+  // barrier (its buffer is free, tile t + 1's is whole) tile t + 1's scores.
+  fetch(0);
+  stash(0);
+  fetch(1);
+  __syncthreads();
+  if (nt > 0) scores(0);
+  for (int t = 0; t < nt; ++t) {
+    fetch(t + 2);
+    __builtin_amdgcn_sched_barrier(0);
+    const u32x4* vs = smem + (t & 1) * BUF + 3 * KU + 2 * hh * NDB * 64 + lu;
+    const int j0 = t * kBK + hh * 32;
+    // A half wholly after the wavefront's queries, or past Sk, adds nothing.
+    if (!(P.causal && j0 > q0w + kQW - 1) && j0 < P.Sk) {
+      // s[e]: key j0 + 8 (e / 4) + 4 hi + e % 4, query qi (log2 domain).
+      const bool edge = (P.causal && j0 + 31 > q0w) || j0 + 32 > P.Sk;
+      if (Mp) {
+#pragma unroll
+        for (int e = 0; e < 16; ++e) s[e] = __builtin_fmaf(mv[e], kLog2e, s[e]);
+      }
+      if (edge) {
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+          const int kj = j0 + 8 * (e >> 2) + 4 * hi + (e & 3);
+          if (kj >= P.Sk || (P.causal && kj > qi)) s[e] = -INFINITY;
+        }
+      }
+      float mt = s[0];
+#pragma unroll
+      for (int e = 1; e < 16; ++e) mt = fmaxf(mt, s[e]);
+      mt = fmaxf(mt, xor32(mt));
+      const float m_new = fmaxf(m_run, mt);
+      const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
+      m_run = m_new;
+      if (__builtin_amdgcn_ballot_w64(alpha != 1.0f)) {  // (NaN counts)
+        l_run *= alpha;
+#pragma unroll
+        for (int db = 0; db < NDB; ++db)
+#pragma unroll
+          for (int e = 0; e < 16; ++e) acc[db][e] *= alpha;
+      }
+      float l0 = 0.f, l1 = 0.f;
+#pragma unroll
+      for (int e = 0; e < 16; e += 2) {
+        s[e] = __builtin_amdgcn_exp2f(s[e] - m_new);
+        s[e + 1] = __builtin_amdgcn_exp2f(s[e + 1] - m_new);
+        l0 += s[e];
+        l1 += s[e + 1];
+      }
+      l_run += l0 + l1;
+      // O^T[32 db + lane % 32][q] += V^T P^T over 16 keys an MFMA: registers
+      // 8 m .. 8 m + 7 are, split and packed, its B operand.
+#pragma unroll
+      for (int m = 0; m < 2; ++m) {
+        float px[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) px[j] = s[8 * m + j];
+        u32x4 pp[3];
+        uint32_t any = bgk::kSplitTop;
+        bgk::split8(px, pp[0], pp[1], pp[2], any);
+#pragma unroll
+        for (int db = 0; db < NDB; ++db) {
+          bgk::bf16x8 vf[3];
+#pragma unroll
+          for (int p = 0; p < 3; ++p)
+            vf[p] = __builtin_bit_cast(bgk::bf16x8, vs[p * VU + (m * NDB + db) * 64]);
+#pragma unroll
+          for (int p = 0; p < 6; ++p)
+            acc[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[QA[p]], __builtin_bit_cast(bgk::bf16x8, pp[QB[p]]),
+                                                             acc[db], 0, 0, 0);
+        }
+      }
+    }
+    __syncthreads();
+    if (t + 1 < nt) scores(t + 1);
+  }
+
+  // The two key halves of a query block merge through LDS.
+  float* red = reinterpret_cast<float*>(smem) + (w & 3) * 64 * 36 + lane;
+  __syncthreads();
+  if (hh == 1) {
+    red[0] = m_run;
+    red[64] = l_run;
+#pragma unroll
+    for (int db = 0; db < NDB; ++db)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) red[(2 + 16 * db + e) * 64] = acc[db][e];
+  }
+  __syncthreads();
+  bool redo = low < bgk::kSplitMin;
+  if (hh == 0) {
+    const float m = fmaxf(m_run, red[0]);
+    const float f0 = __builtin_amdgcn_exp2f(m_run - m), f1 = __builtin_amdgcn_exp2f(red[0] - m);
+    l_run = l_run * f0 + red[64] * f1;
+#pragma unroll
+    for (int db = 0; db < NDB; ++db)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        acc[db][e] = acc[db][e] * f0 + red[(2 + 16 * db + e) * 64] * f1;
+        redo |= !(fabsf(acc[db][e]) <= 3.402823466e38f);
+      }
+  }
+  const int64_t ohead = int64_t(b) * P.o_sb + int64_t(h) * P.o_sh;
+  const float lt = l_run + xor32(l_run);
+  const float inv = lt > 0.f ? 1.0f / lt : 0.f;
+  redo |= hh == 0 && !(lt <= 3.402823466e38f);
+  // A value that the parts cannot hold may sit in a tile any thread staged.
+  redo = __syncthreads_or(redo);
+  if (hh == 1) return;
+  if (redo) {
+    fa32_plain(P, Qp, Kp, Vp, Mp, ohead, q0w);
+    return;
+  }
+  if (qi >= P.Sq) return;
+#pragma unroll
+  for (int db = 0; db < NDB; ++db)
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+      const int d = 32 * db + 8 * (e >> 2) + 4 * hi + (e & 3);
+      if (d < P.D) bgk::store_from_f32(P.o, P.out_dtype, ohead + int64_t(qi) * P.o_ss + d, acc[db][e] * inv);
+    }
+}
+
+}  // namespace
 namespace bg {
 
 // 16-byte loads of Q, K and V rows: D % 4 == 0, strides in whole 16-byte
@@ -293,6 +646,16 @@ static bool fa32_vec(const bg_attention_desc& d, bool ptrs_aligned) {
 bool fa32_supported(const bg_attention_desc& d) {
   return d.in_dtype == BG_F32 && d.d >= 1 && d.d <= 64 && d.batch * d.heads <= 0x7fffffff &&
          d.sq <= int64_t(65535) * kBQ && d.sk <= (int64_t(1) << 30) && d.sq <= (int64_t(1) << 30);
+}
+
+// The split kernel from two key tiles on (one tile: 16 queries and keys 10.2
+// against 8.7 us, 64: 11.5 against 11.3); K and V of a head within a 32-bit
+// buffer offset.
+static bool fa32_split(const bg_attention_desc& d) {
+  const int64_t lim = int64_t(1) << 31;
+  return d.reserved != BG_ATTENTION_TILED && d.sk > kBK && ((d.sk - 1) * d.k_ss + d.d) * 4 < lim &&
+         ((d.sk - 1) * d.v_ss + d.d) * 4 < lim && (d.sk + 2 * kBK) * d.k_ss * 4 < 2 * lim &&
+         (d.sk + 2 * kBK) * d.v_ss * 4 < 2 * lim;
 }
 
 // q, k, v, o point at the first element of each operand (offsets applied);
@@ -323,9 +686,19 @@ void launch_fa32(bg_ctx* ctx, const bg_attention_desc& d, const float* q, const 
   const bool vec = fa32_vec(d, al16(q) && al16(k) && al16(v));
   const dim3 grid(unsigned(d.batch * d.heads), unsigned(A.n_qblocks), 1);
   auto go = [&](auto kern) { dispatch(ctx, kern, grid, dim3(kNW * 64), 0, A); };
-  if (d.d <= 16) vec ? go(fa32_fwd_kernel<16, true>) : go(fa32_fwd_kernel<16, false>);
-  else if (d.d <= 32) vec ? go(fa32_fwd_kernel<32, true>) : go(fa32_fwd_kernel<32, false>);
-  else vec ? go(fa32_fwd_kernel<64, true>) : go(fa32_fwd_kernel<64, false>);
+  if (fa32_split(d)) {
+    const uint32_t kb = uint32_t(((d.sk - 1) * d.k_ss + d.d) * 4), vb = uint32_t(((d.sk - 1) * d.v_ss + d.d) * 4);
+    auto sgo = [&](auto kern) { dispatch(ctx, kern, grid, dim3(kSplitNT), 0, A, kb, vb); };
+    if (d.d <= 16) vec ? sgo(split_fa32_fwd_kernel<16, true>) : sgo(split_fa32_fwd_kernel<16, false>);
+    else if (d.d <= 32) vec ? sgo(split_fa32_fwd_kernel<32, true>) : sgo(split_fa32_fwd_kernel<32, false>);
+    else vec ? sgo(split_fa32_fwd_kernel<64, true>) : sgo(split_fa32_fwd_kernel<64, false>);
+  } else if (d.d <= 16) {
+    vec ? go(fa32_fwd_kernel<16, true>) : go(fa32_fwd_kernel<16, false>);
+  } else if (d.d <= 32) {
+    vec ? go(fa32_fwd_kernel<32, true>) : go(fa32_fwd_kernel<32, false>);
+  } else {
+    vec ? go(fa32_fwd_kernel<64, true>) : go(fa32_fwd_kernel<64, false>);
+  }
   hip_check(hipGetLastError(), "f32 attention launch");
 }
 
@@ -379,15 +752,17 @@ void plan_attention(const bg_attention_desc& d0, bg_launch_plan& out) {
   out.k_slices = 1;
   out.lds_bytes = 2 * 2 * kBK * 16 * 16;
   out.n_launches = 1;
+  const bool split = fa32_split(d);
+  if (split) out.lds_bytes = std::max(2 * 3 * 16 * (dp * 8 + (dp > 32 ? 512 : 256)), 4 * 64 * 9 * 16);
   bg_launch_plan_entry& e = out.launch[0];
-  std::snprintf(e.family, sizeof e.family, "%s", "fa32_fwd_kernel");
+  std::snprintf(e.family, sizeof e.family, "%s", split ? "split_fa32_fwd_kernel" : "fa32_fwd_kernel");
   e.n_targs = 2;
   e.targs[0] = dp;
   e.targs[1] = fa32_vec(d, ptrs) ? 1 : 0;
   e.grid[0] = d.batch * d.heads;
   e.grid[1] = (d.sq + kBQ - 1) / kBQ;
   e.grid[2] = 1;
-  e.block[0] = kNW * 64; e.block[1] = 1; e.block[2] = 1;
+  e.block[0] = split ? kSplitNT : kNW * 64; e.block[1] = 1; e.block[2] = 1;
 }
 
 }  // namespace bg

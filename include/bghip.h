@@ -230,8 +230,9 @@ typedef struct bg_attention_desc {
   int32_t reserved;     /* 0, or BG_ATTENTION_TILED */
 } bg_attention_desc;
 
-/* In `reserved`: calls of a few query rows, which by default stream K
- * and V without matrix instructions, run the tiled kernels as well. */
+/* In `reserved`: calls of a few query rows, which by default stream K and V
+ * without matrix instructions, run the tiled kernels as well, and f32 calls
+ * form every product by a float32 matrix instruction. */
 #define BG_ATTENTION_TILED 1
 
 /* Resource snapshot (realizer.ts:287-298 WebGpuResourceSnapshot). */

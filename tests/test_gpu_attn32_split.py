@@ -1,0 +1,127 @@
+"""float32 attention on the bf16 matrix core (three bf16 parts of each value):
+against float64 and the float32 kernel, the launch plan, and the values the
+parts cannot hold."""
+import numpy as np
+import pytest
+
+from browsergrad_amd import _native as N
+
+pytestmark = pytest.mark.gpu
+F32 = np.float32
+
+
+@pytest.fixture(scope="module")
+def bridge():
+    from browsergrad_amd.bridge import HipRealizerBridge
+    with HipRealizerBridge(device=0) as br:
+        yield br
+
+
+def _run(br, hs, **kw):
+    br.set_launch_log(True)
+    br.take_launch_log()
+    h = br.attention_ex(*hs, in_dtype="float32", out_dtype="float32", **kw)
+    log = br.take_launch_log()
+    br.set_launch_log(False)
+    y = br.to_numpy(h)
+    br.release(h)
+    return y, log
+
+
+def _truth(q, k, v, scale, causal):
+    q, k, v = (x.astype(np.float64) for x in (q, k, v))
+    with np.errstate(all="ignore"):
+        s = q @ k.transpose(0, 1, 3, 2) * scale
+        if causal:
+            s = np.where(np.triu(np.ones(s.shape[-2:], bool), 1), -np.inf, s)
+        p = np.exp(s - s.max(-1, keepdims=True))
+        p /= p.sum(-1, keepdims=True)
+        return p @ v, p @ np.abs(v)
+
+
+# Two tiles and more, ragged key and query counts, more queries than keys, every
+# padded head dim, odd head dims (4-byte loads), one workgroup and many.
+@pytest.mark.parametrize("b,h,sq,sk,d", [(1, 1, 5, 65, 64), (2, 3, 128, 128, 16), (1, 2, 130, 200, 64), (1, 2, 300, 97, 32),
+                                         (2, 2, 64, 200, 7), (1, 1, 257, 257, 33), (4, 12, 1000, 1000, 64),
+                                         (1, 3, 31, 1025, 48), (3, 1, 96, 128, 24)])
+@pytest.mark.parametrize("causal", [False, True])
+def test_split_attention(bridge, b, h, sq, sk, d, causal):
+    rng = np.random.default_rng(sq + sk + d)
+    q, k, v = (rng.standard_normal((b, h, n, d)).astype(F32) for n in (sq, sk, sk))
+    hs = [bridge.upload(t, t.shape, "float32") for t in (q, k, v)]
+    kw = dict(batch=b, heads=h, sq=sq, sk=sk, d=d, scale=d ** -0.5, causal=causal)
+    y, log = _run(bridge, hs, **kw)
+    from browsergrad_amd.semantic import launch_plan
+    a = N.AttentionDesc()
+    a.batch, a.heads, a.sq, a.sk, a.d, a.causal = b, h, sq, sk, d, int(causal)
+    a.in_dtype = a.out_dtype = N.BG_F32
+    plan = launch_plan("attention", a)["launches"]
+    assert "split_fa32_fwd_kernel" in log[0]["kernel"] and plan[0]["family"] == "split_fa32_fwd_kernel"
+    assert [(r["grid"], r["block"]) for r in log] == [(e["grid"], e["block"]) for e in plan]
+    truth, mass = _truth(q, k, v, d ** -0.5, causal)
+    # scores carry sqrt(D) roundings of |q||k|/sqrt(D) (about 1e-6), sums sqrt(Sk)
+    assert np.all(np.abs(y - truth) <= (4e-6 + 2.0 * np.sqrt(sk) * 2.0 ** -24) * mass)
+    old, log = _run(bridge, hs, tiled=True, **kw)
+    assert "split" not in log[0]["kernel"]
+    err = [np.linalg.norm(t - truth) / np.linalg.norm(truth) for t in (y, old)]
+    assert err[0] <= 1.05 * err[1] + 2.0 ** -25, err
+    for x in hs:
+        bridge.release(x)
+
+
+def test_split_attention_mask_and_views(bridge):
+    """An additive mask (with a row of -inf, which gives zeros) and Q, K, V as
+    views of one projection with an odd head dim."""
+    b, h, s, d = 2, 3, 150, 64
+    rng = np.random.default_rng(2)
+    q, k, v = (rng.standard_normal((b, h, s, d)).astype(F32) for _ in range(3))
+    mask = rng.uniform(-0.5, 0.5, (b, 1, s, s)).astype(F32)
+    mask[rng.random(mask.shape) < 0.05] = -np.inf
+    mask[:, :, 5] = -np.inf
+    hs = [bridge.upload(t, t.shape, "float32") for t in (q, k, v, mask)]
+    y = bridge.to_numpy(bridge.flash_attention(*hs, b, h, s, s, d, 0.125, "float32"))
+    sc = q.astype(np.float64) @ k.astype(np.float64).transpose(0, 1, 3, 2) * 0.125 + mask
+    m = sc.max(-1, keepdims=True)
+    p = np.exp(sc - np.where(np.isfinite(m), m, 0))
+    truth = p @ v.astype(np.float64) / np.where(m == -np.inf, 1, p.sum(-1, keepdims=True))
+    assert np.all(y[:, :, 5] == 0) and np.max(np.abs(y - truth)) <= 2e-5
+    B, S, H, D = 2, 150, 3, 21
+    x = rng.standard_normal((B, S, 3, H, D)).astype(F32)
+    hx = bridge.upload(x, x.shape, "float32")
+    st = (S * 3 * H * D, D, 3 * H * D)
+    y, log = _run(bridge, (hx, hx, hx), batch=B, heads=H, sq=S, sk=S, d=D, scale=0.3, causal=True, q_view=(0, *st),
+                  k_view=(H * D, *st), v_view=(2 * H * D, *st), o_strides=(S * H * D, D, H * D))
+    assert "split_fa32_fwd_kernel" in log[0]["kernel"]
+    truth, mass = _truth(*(np.ascontiguousarray(x[:, :, i].transpose(0, 2, 1, 3)) for i in range(3)), 0.3, True)
+    assert np.all(np.abs(y.reshape(B, S, H, D).transpose(0, 2, 1, 3) - truth) <= 1e-5 * mass)
+
+
+@pytest.mark.parametrize("what", ["nan_k", "inf_v", "neg_inf_k", "tiny_v", "tiny_k", "huge_q"])
+def test_split_attention_special_values(bridge, what):
+    """What the parts cannot hold gives what the float32 kernel gives."""
+    rng = np.random.default_rng(8)
+    b, h, s, d = 1, 2, 140, 64
+    q, k, v = (rng.standard_normal((b, h, s, d)).astype(F32) for _ in range(3))
+    if what == "nan_k":
+        k[0, 0, 70, 3] = np.nan
+    elif what == "inf_v":
+        v[0, 1, 3, 7] = np.inf
+    elif what == "neg_inf_k":
+        q[..., 0], k[0, 0, 9, 0] = 1, -np.inf
+    elif what == "tiny_v":
+        v[0, 0] *= F32(2.0 ** -130)
+    elif what == "tiny_k":
+        k[0, 0] *= F32(2.0 ** -120)
+    else:
+        q[0, 0, 4] *= F32(3e37)
+    hs = [bridge.upload(t, t.shape, "float32") for t in (q, k, v)]
+    kw = dict(batch=b, heads=h, sq=s, sk=s, d=d, scale=0.125)
+    y, log = _run(bridge, hs, **kw)
+    t, _ = _run(bridge, hs, tiled=True, **kw)
+    assert "split_fa32_fwd_kernel" in log[0]["kernel"]
+    assert np.array_equal(np.isnan(y), np.isnan(t)) and np.array_equal(np.isposinf(y), np.isposinf(t))
+    fin = np.isfinite(t)
+    _, mass = _truth(q, k, np.where(np.isfinite(v), v, 0), 0.125, False)
+    if what != "huge_q":  # (scores of 1e37 round to 1e30: any order of their sum picks the same key only by luck)
+        ok = fin & np.isfinite(mass)
+        assert np.all(np.abs(y[ok].astype(np.float64) - t[ok]) <= 2e-5 * mass[ok] + 2.0 ** -148)
