@@ -25,6 +25,7 @@
 
 #include "common.cuh"
 #include "core.h"
+#include "split.cuh"
 
 namespace {
 
@@ -363,6 +364,254 @@ __global__ void __launch_bounds__(256) conv_gemm_kernel(ConvK P) {
   }
 
   conv_epilogue<MODE, BM, BN>(P, acc, m0, n0, wm, wn, g, split, P.M);
+}
+
+// ---- weight gradient on the bf16 matrix core -----------------------------------------
+//
+// WGRAD with every float32 value as three bf16 parts (split.cuh): the ring of
+// three 16-deep stages, the two sets of sums and the float32 redo are those of
+// gemm32_split_kernel; both operands pass through registers here.  dy: lanes
+// 2 r and 2 r + 1 read eight consecutive positions of row r each (two 16-byte
+// loads where an image holds a multiple of eight).  x: the 64 columns (c, tap)
+// of a wavefront take the same eight positions, which the scalar unit
+// decomposes; they end at most one row (oW >= 8), so a column keeps the offsets
+// of two rows and adds its position's.
+//
+// Bound by x's gathers (a load's 64 lanes touch about seven channels' three
+// rows) beside the matrix core.  Measured, with the sum over the slices: 32 x
+// 128 x 28 x 28 with 128 3x3 filters 115 -> 73 us (its 44 GFLOP of bf16
+// products take 37 us at 1.2 PFLOP/s), 32 x 64 x 56 x 56 163 -> 112, 64 x 256 x
+// 14 x 14 204 -> 154; error against 64 bits 3.5e-7 -> 1.8e-7.
+template <int BM, int WGM, int WGN>
+__global__ void __launch_bounds__(256, 2)
+    conv_wgrad_split_kernel(ConvK P, uint32_t a_bytes, uint32_t b_bytes, int a16) {
+  constexpr int BN = 128, NT = 256;
+  constexpr int TM = BM / WGM / 32, TN = BN / WGN / 32;
+  constexpr int UA = 2 * BM, UB = 2 * BN;  // 16-byte units per plane
+  constexpr int STAGE = 3 * (UA + UB);
+  static_assert(TM >= 2 && WGM * WGN == 4, "a step splits dy beside its first row group and x beside its second");
+  typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+  __shared__ u32x4 smem[3 * STAGE];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave / WGN, wn = wave % WGN;
+  const int tm = int(blockIdx.x) % P.tiles_m, tn = int(blockIdx.x) / P.tiles_m;
+  const int g = int(blockIdx.y) / P.ksplit, split = int(blockIdx.y) % P.ksplit;
+  const int m0 = tm * BM, n0 = tn * BN;
+  const int kbeg = split * P.k_chunk, kend = min(P.K, kbeg + P.k_chunk);
+  const int nk = (kend - kbeg + 15) / 16;
+  const int HW = P.H * P.W, oHW = P.oH * P.oW, KHW = P.KH * P.KW;
+  constexpr uint32_t kOut = 0x80000000u;
+  const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc((void*)P.a, (short)0, int(a_bytes), 0x00020000);
+  const __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc((void*)P.b, (short)0, int(b_bytes), 0x00020000);
+
+  // dy unit: row tid / 2, chunk tid % 2.  x unit: column tid % 128, chunk tid / 128.
+  const int ar = tid >> 1, ac = tid & 1;
+  const bool a_in = UA >= NT || tid < UA;
+  const uint32_t a_row = a_in && m0 + ar < P.M ? uint32_t((g * P.Opg + m0 + ar) * P.oS) * 4 : kOut;
+  const int wa = (ar >> 5) * 64 + ac * 32 + ((ar & 31) ^ (ac * 8));
+  const int bc = tid & 127, bk = __builtin_amdgcn_readfirstlane(tid >> 7);
+  const int wb = (bc >> 5) * 64 + bk * 32 + ((bc & 31) ^ (bk * 8));
+  const int j = n0 + bc;
+  const uint32_t jj = j < P.NC ? uint32_t(j) : 0u;
+  const uint32_t c = fdiv(jj, P.f_KV), kv = jj - c * uint32_t(P.KV);
+  const uint32_t kd = fdiv(kv, P.f_KHW), kr = kv - kd * uint32_t(KHW);
+  const uint32_t kh = fdiv(kr, P.f_KW), kw = kr - kh * uint32_t(P.KW);
+  const uint32_t b_chan = j < P.NC ? uint32_t((g * P.Cpg + int(c)) * P.S) * 4 : kOut;
+  const int b_d = int(kd) * P.dd - P.pd, b_h = int(kh) * P.dh - P.ph, b_w = int(kw) * P.dw - P.pw;
+
+  float xa[8], xb[8];
+  uint32_t low = kSplitTop;
+  // Byte offset of x's row for output row (n, od, oh), high bit set outside.
+  auto x_row = [&](uint32_t n, uint32_t od, uint32_t oh, bool in) {
+    const int id = int(od) * P.sd + b_d, ih = int(oh) * P.sh + b_h;
+    const bool ok = in && unsigned(id) < unsigned(P.D) && unsigned(ih) < unsigned(P.H);
+    return (b_chan + (n * uint32_t(P.C * P.S) + uint32_t(id * HW + ih * P.W)) * 4) | (ok ? b_chan & kOut : kOut);
+  };
+  auto load_stage = [&](int t) {
+    const int k0 = kbeg + t * 16;
+    {
+      const uint32_t k = uint32_t(k0 + 8 * ac);
+      const uint32_t n = fdiv(k, P.f_oS), sp = k - n * uint32_t(P.oS);
+      const uint32_t off = a_row + (n * uint32_t(P.O) * uint32_t(P.oS) + sp) * 4;
+      if (a16) {
+        const uint32_t at = off | (a_row & kOut) | (int(k) < kend ? 0u : kOut);
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(ra, at + 16 * h, 0, 0);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) xa[4 * h + e] = __uint_as_float(v[e]);
+        }
+      } else {
+        uint32_t at = off, s = sp;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          xa[e] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
+              ra, at | (a_row & kOut) | (int(k) + e < kend ? 0u : kOut), 0, 0));
+          const bool wrap = ++s == uint32_t(P.oS);  // the next position is the next image's first
+          at += wrap ? uint32_t((P.O - 1) * P.oS + 1) * 4 : 4u;
+          s = wrap ? 0u : s;
+        }
+      }
+    }
+    const uint32_t k = uint32_t(k0 + 8 * bk);  // uniform
+    const uint32_t n = fdiv(k, P.f_oS), sp = k - n * uint32_t(P.oS);
+    const uint32_t od = fdiv(sp, P.f_oHW), r = sp - od * uint32_t(oHW);
+    const uint32_t oh = fdiv(r, P.f_oW), ow = r - oh * uint32_t(P.oW);
+    const uint32_t kn = k - ow + uint32_t(P.oW);  // first position of the next row
+    const uint32_t n1 = fdiv(kn, P.f_oS), sp1 = kn - n1 * uint32_t(P.oS);
+    const uint32_t od1 = fdiv(sp1, P.f_oHW), oh1 = fdiv(sp1 - od1 * uint32_t(oHW), P.f_oW);
+    const uint32_t r0 = x_row(n, od, oh, int(k) < kend), r1 = x_row(n1, od1, oh1, int(kn) < kend);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const uint32_t q = ow + e;  // uniform, as is the choice of the row
+      const bool next = q >= uint32_t(P.oW);
+      const int iw = int(next ? q - uint32_t(P.oW) : q) * P.sw + b_w;
+      const uint32_t row = next ? r1 : r0;
+      const bool ok = unsigned(iw) < unsigned(P.W) && int(k) + e < kend;
+      xb[e] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
+          rb, (row + uint32_t(iw) * 4) | (row & kOut) | (ok ? 0u : kOut), 0, 0));
+    }
+  };
+  auto put = [&](u32x4* st, int plane, const float (&x)[8]) {
+    u32x4 p1, p2, p3;
+    split8(x, p1, p2, p3, low);
+    st[0] = p1;
+    st[plane] = p2;
+    st[2 * plane] = p3;
+  };
+  auto put_a = [&](int slot) {
+    if (UA >= NT || wave * 64 < UA) put(smem + slot * STAGE + wa, UA, xa);
+  };
+  auto put_b = [&](int slot) { put(smem + slot * STAGE + 3 * UA + wb, UB, xb); };
+
+  const int lu = lane ^ ((lane >> 5) << 3);
+  bf16x8 fa[2][3], fb[3][TN];
+  auto read_a = [&](int slot, int i, bf16x8 (&f)[3]) {
+#pragma unroll
+    for (int q = 0; q < 3; ++q)
+      f[q] = __builtin_bit_cast(bf16x8, smem[slot * STAGE + q * UA + (wm * TM + i) * 64 + lu]);
+  };
+  auto read_b = [&](int slot, int q) {
+#pragma unroll
+    for (int i = 0; i < TN; ++i)
+      fb[q][i] = __builtin_bit_cast(bf16x8, smem[slot * STAGE + 3 * UA + q * UB + (wn * TN + i) * 64 + lu]);
+  };
+  float16v acc[TM][TN], small[TM][TN];
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int jt = 0; jt < TN; ++jt)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) acc[i][jt][e] = small[i][jt][e] = 0.f;
+  auto mul = [&](int i, int qa, int qb) {
+#pragma unroll
+    for (int jt = 0; jt < TN; ++jt) {
+      float16v& d = qa + qb > 0 ? small[i][jt] : acc[i][jt];
+      d = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[i & 1][qa], fb[qb][jt], d, 0, 0, 0);
+    }
+  };
+  load_stage(0);
+  put_a(0);
+  put_b(0);
+  load_stage(1);  // (past the last stage every load is out of range: zeros)
+  put_a(1);
+  put_b(1);
+  load_stage(2);
+  __syncthreads();
+  read_a(0, 0, fa[0]);
+#pragma unroll
+  for (int q = 0; q < 3; ++q) read_b(0, q);
+  // One barrier a step, after the first row group's MFMAs: the slot of stage
+  // t - 1 is free for stage t + 2 and stage t + 1 may be read.
+  int slot = 0;
+  for (int t = 0; t < nk; ++t) {
+    const int nslot = slot == 2 ? 0 : slot + 1, wslot = slot == 0 ? 2 : slot - 1;
+#pragma unroll
+    for (int i = 0; i < TM; ++i) {
+      const bool last = i + 1 == TM;
+      if (!last) read_a(slot, i + 1, fa[(i + 1) & 1]);
+      else read_a(nslot, 0, fa[(i + 1) & 1]);
+      mul(i, 2, 0);
+      mul(i, 0, 2);
+      if (last) read_b(nslot, 2);
+      mul(i, 1, 1);
+      mul(i, 0, 1);
+      if (last) read_b(nslot, 1);
+      mul(i, 1, 0);
+      mul(i, 0, 0);
+      if (last) read_b(nslot, 0);
+      if (i == 0) {
+        __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
+        __builtin_amdgcn_s_barrier();
+        put_a(wslot);
+      }
+      if (i == 1) {
+        put_b(wslot);
+        load_stage(t + 3);
+      }
+    }
+    slot = nslot;
+  }
+
+  bool redo = low < kSplitMin;
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int jt = 0; jt < TN; ++jt) {
+      acc[i][jt] += small[i][jt];
+#pragma unroll
+      for (int e = 0; e < 16; ++e) redo |= !(fabsf(acc[i][jt][e]) <= 3.402823466e38f);
+    }
+  if (__syncthreads_or(redo)) {
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int jt = 0; jt < TN; ++jt)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) acc[i][jt][e] = 0.f;
+    for (int k = kbeg; k < kend; k += 2) {  // float32 MFMAs: k = lane / 32 on both operands
+      const bool k_ok = k + (lane >> 5) < kend;
+      const uint32_t ke = k_ok ? uint32_t(k + (lane >> 5)) : 0u;
+      const uint32_t n = fdiv(ke, P.f_oS), sp = ke - n * uint32_t(P.oS);
+      const uint32_t od = fdiv(sp, P.f_oHW), r = sp - od * uint32_t(oHW);
+      const uint32_t oh = fdiv(r, P.f_oW), ow = r - oh * uint32_t(P.oW);
+      float b[TN];
+#pragma unroll
+      for (int jt = 0; jt < TN; ++jt) {
+        const int col = n0 + wn * (BN / WGN) + jt * 32 + (lane & 31);
+        const uint32_t cc = col < P.NC ? uint32_t(col) : 0u;
+        const uint32_t ch = fdiv(cc, P.f_KV), v = cc - ch * uint32_t(P.KV);
+        const uint32_t vd = fdiv(v, P.f_KHW), vr = v - vd * uint32_t(KHW);
+        const uint32_t vh = fdiv(vr, P.f_KW), vw = vr - vh * uint32_t(P.KW);
+        const int id = int(od) * P.sd + int(vd) * P.dd - P.pd, ih = int(oh) * P.sh + int(vh) * P.dh - P.ph,
+                  iw = int(ow) * P.sw + int(vw) * P.dw - P.pw;
+        const bool ok = k_ok && col < P.NC && unsigned(id) < unsigned(P.D) && unsigned(ih) < unsigned(P.H) &&
+                        unsigned(iw) < unsigned(P.W);
+        b[jt] = ok ? P.b[(int64_t(n) * P.C + g * P.Cpg + ch) * P.S + (int64_t(id) * P.H + ih) * P.W + iw] : 0.f;
+      }
+#pragma unroll
+      for (int i = 0; i < TM; ++i) {
+        const int row = m0 + wm * (BM / WGM) + i * 32 + (lane & 31);
+        const float a = k_ok && row < P.M ? P.a[(int64_t(n) * P.O + g * P.Opg + row) * P.oS + sp] : 0.f;
+#pragma unroll
+        for (int jt = 0; jt < TN; ++jt)
+          acc[i][jt] = __builtin_amdgcn_mfma_f32_32x32x2f32(a, b[jt], acc[i][jt], 0, 0, 0);
+      }
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int jt = 0; jt < TN; ++jt) {
+      const int col = n0 + wn * (BN / WGN) + jt * 32 + (lane & 31);
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        const int row = m0 + wm * (BM / WGM) + i * 32 + 8 * (e >> 2) + 4 * (lane >> 5) + (e & 3);
+        if (row < P.M && col < P.NC)
+          P.out[int64_t(split) * P.part_stride + (int64_t(g) * P.Opg + row) * P.NC + col] = acc[i][jt][e];
+      }
+    }
 }
 
 // Forward convolution with the operands gathered straight into an S-stage
@@ -1098,6 +1347,14 @@ void launch_conv(bg_ctx* ctx, const ConvProblem& p, int mode, const float* a, co
   int bm = k.M >= 128 ? 128 : 64;
   int bn = k.NC >= 128 ? 128 : 64;
   if (mode != 2 && ((k.M + bm - 1) / bm) * int64_t((k.NC + bn - 1) / bn) * G < 512) bm = bn = 64;
+  // Weight gradient from bf16 parts, on the same tiles: 128 columns (with 64
+  // half of x's work is padding: 1x1 over 64 channels 32 -> 34 us), rows of
+  // eight positions at least (below, each position finds its own row: 128 x 64
+  // x 6 x 6 23 -> 25 us), eight steps (under them the ring never fills: 8 x 8
+  // images of 16 channels 9.4 -> 10.4 us; 12 x 12 17.2 -> 15.7) and operands
+  // that 31-bit byte offsets reach.
+  const bool wsplit = mode == 2 && bn == 128 && k.oW >= 8 && k.K >= 8 * CBK &&
+                      p.n * int64_t(k.O) * k.oS < (int64_t(1) << 29) && p.n * int64_t(k.C) * k.S < (int64_t(1) << 29);
   k.tiles_m = int((k.M + bm - 1) / bm);
   const int64_t tiles_n = (k.NC + bn - 1) / bn;
   const int64_t tiles = int64_t(k.tiles_m) * tiles_n;
@@ -1108,9 +1365,12 @@ void launch_conv(bg_ctx* ctx, const ConvProblem& p, int mode, const float* a, co
     // slices it holds times the slice length: on the ResNet 3x3 layers the
     // former rule (1024 workgroups, at most 64 slices) and a 512-workgroup
     // one each lose 5-20% somewhere (e.g. 32 x 128 x 28 x 28: 145 / 124 /
-    // 119 us; 128 x 512 x 7 x 7: 406 / 491 / 400 us).
+    // 119 us; 128 x 512 x 7 x 7: 406 / 491 / 400 us).  The split kernel, two
+    // workgroups per CU by its LDS, takes 512 (256 / 512 / 768: 95 / 73 / 83
+    // us on the former layer, 153 / 112 / 141 on 32 x 64 x 56 x 56).
     const int64_t steps = (int64_t(k.K) + CBK - 1) / CBK;
-    int64_t splits = std::max<int64_t>(1, std::min<int64_t>(768 / std::max<int64_t>(tiles * G, 1), steps / 8));
+    const int64_t want = (wsplit ? 512 : 768) / std::max<int64_t>(tiles * G, 1);
+    int64_t splits = std::max<int64_t>(1, std::min<int64_t>(want, steps / 8));
     splits = std::min<int64_t>(splits, 128);
     splits = std::min<int64_t>(splits, 65535 / G);
     const int64_t chunk_steps = (steps + splits - 1) / std::max<int64_t>(splits, 1);
@@ -1126,6 +1386,17 @@ void launch_conv(bg_ctx* ctx, const ConvProblem& p, int mode, const float* a, co
   }
   if (k.M == 0 || k.NC == 0) return;
   const dim3 grid(unsigned(tiles), unsigned(G * k.ksplit));
+  if (wsplit) {
+    const uint32_t ab = uint32_t(p.n * int64_t(k.O) * k.oS * 4), bb = uint32_t(p.n * int64_t(k.C) * k.S * 4);
+    const int a16 = k.oS % 8 == 0 && (reinterpret_cast<uintptr_t>(a) & 15) == 0;
+    auto go = [&](auto kern) { dispatch(ctx, kern, grid, dim3(256), 0, k, ab, bb, a16); };
+    bm == 128 ? go(conv_wgrad_split_kernel<128, 2, 2>) : go(conv_wgrad_split_kernel<64, 1, 4>);
+    if (k.ksplit > 1)
+      dispatch(ctx, conv_split_reduce_kernel, dim3(unsigned((k.part_stride + 255) / 256)), dim3(256), 0, k.out, out,
+               k.part_stride, k.ksplit);
+    hip_check(hipGetLastError(), "conv launch");
+    return;
+  }
   // Forward: the LDS-ring kernel when x and w fit 32-bit byte offsets
   // (BG_CONV_RING=0 selects the register-staged kernel, for comparisons).
   const int64_t a_bytes = p.n * int64_t(k.C) * k.S * 4, b_bytes = int64_t(k.O) * k.K * 4;
