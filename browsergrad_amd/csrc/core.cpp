@@ -215,6 +215,12 @@ void* scratch(bg_ctx* ctx, size_t bytes, int slot) {
   return ctx->scratch[slot];
 }
 
+bool stream_capturing(bg_ctx* ctx) {
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  hip_check(hipStreamIsCapturing(ctx->stream, &st), "hipStreamIsCapturing");
+  return st != hipStreamCaptureStatusNone;
+}
+
 static hipEvent_t take_event(bg_ctx* ctx) {
   if (!ctx->event_pool.empty()) {
     hipEvent_t e = ctx->event_pool.back();

@@ -116,6 +116,10 @@ bg_handle mint_view(bg_ctx* ctx, const Record& src, int64_t offset,
                     int64_t nbytes, const std::vector<int64_t>& shape,
                     int dtype);
 void* scratch(bg_ctx* ctx, size_t bytes, int slot = 0);
+// True while the context's stream is captured into a graph: a later call may
+// grow (free) a scratch slot that the graph still names, so a call that can
+// do without partials then takes one slice.
+bool stream_capturing(bg_ctx* ctx);
 std::vector<int64_t> to_shape(const int64_t* shape, int rank);
 int64_t numel(const std::vector<int64_t>& shape);
 

@@ -235,7 +235,8 @@ namespace bg {
 int attention_decode_slices(const bg_attention_desc& d, bool ptrs_aligned) {
   if (d.in_dtype != BG_F32 && d.in_dtype != BG_F16 && d.in_dtype != BG_BF16) return 0;
   const int64_t es = dtype_size(d.in_dtype), e = 16 / es;
-  if (!ptrs_aligned || d.sq > (d.in_dtype == BG_F32 ? 4 : 2) || d.sk < 64 || d.sk > (int64_t(1) << 30) || d.d > 64 || d.d % e != 0 ||
+  if (!ptrs_aligned || d.sq > (d.in_dtype == BG_F32 ? 4 : 2) || d.sk < 64 ||
+      d.sk > (int64_t(1) << 30) || d.d > 64 || d.d % e != 0 ||
       d.batch * d.heads > 0x7fffffff || d.reserved == BG_ATTENTION_TILED)
     return 0;
   for (int64_t s : {d.q_sb, d.q_sh, d.q_ss, d.k_sb, d.k_sh, d.k_ss, d.v_sb, d.v_sh, d.v_ss})
@@ -249,8 +250,9 @@ int attention_decode_slices(const bg_attention_desc& d, bool ptrs_aligned) {
 bool launch_attention_decode(bg_ctx* ctx, const bg_attention_desc& d, const char* q, const char* k, const char* v,
                              void* o) {
   auto al16 = [](const char* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
-  const int slices = attention_decode_slices(d, al16(q) && al16(k) && al16(v));
+  int slices = attention_decode_slices(d, al16(q) && al16(k) && al16(v));
   if (slices == 0) return false;
+  if (slices > 1 && stream_capturing(ctx)) slices = 1;
   DecArgs A{};
   A.q = q;
   A.k = k;
