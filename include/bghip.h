@@ -167,7 +167,7 @@ typedef struct bg_matmul_desc {
   int64_t stride_a, stride_b, stride_c;  /* batch strides in elements (0 = broadcast) */
   int64_t offset_a, offset_b;            /* element offsets into a / b */
   int32_t trans_b;
-  int32_t in_dtype;      /* BG_F32 (f32 MFMA) / BG_F16 / BG_BF16 */
+  int32_t in_dtype;      /* BG_F32 / BG_F16 / BG_BF16 */
   int32_t out_dtype;     /* BG_F32 / BG_F16 / BG_BF16 */
   int32_t round_f16;     /* round accumulator to the intermediate dtype before bias */
   int32_t act;           /* BG_ACT_* */
