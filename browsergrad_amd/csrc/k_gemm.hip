@@ -1075,7 +1075,7 @@ static void run_gemm(bg_ctx* ctx, const bg_matmul_desc& d, const char* a, const 
     const bool aligned = g.aligned;
     Profile prof(ctx, "gemm_f32", bytes, flops);
     const size_t room = workspace_room(ws);
-    const bool skinny = aligned && skinny_plan(d, BG_F32, room).on;
+    const bool skinny = !g.wide && aligned && skinny_plan(d, BG_F32, room).on;
     Gemm32Split gs = gemm32_split(d, g.wide, skinny, room);
     if (gs.slices > 1 && !ws.fixed && stream_capturing(ctx)) gs = gemm32_split(d, g.wide, skinny, 0);
     if (gs.tile >= 0) {

@@ -293,16 +293,16 @@ constexpr Tile kTiles[] = {
 };
 constexpr int64_t kMaxPartials = int64_t(64) << 20;
 
-// Time of m x n x k with `slices` K slices: rounds of workgroups, each about
+// Time of `tiles` tiles of m x n values in all and k with `slices` K slices: rounds of workgroups, each about
 // three steps longer than its k for the first loads and the epilogue, 3 us of
 // launch, and for slices a second launch and the partials' way to memory and
 // back.
-double model_us(const Tile& t, int64_t m, int64_t n, int64_t k, int64_t batch, int slices) {
-  const int64_t steps = (k + 16 * slices - 1) / (16 * slices);
-  const int64_t wgs = (m + t.bm - 1) / t.bm * ((n + t.bn - 1) / t.bn) * batch * slices;
+double model_us(const Tile& t, int64_t tiles, int64_t mn, uint32_t k, uint32_t slices) {
+  const uint32_t steps = (k + 16 * slices - 1) / (16 * slices);
+  const int64_t wgs = tiles * slices;
   const int64_t slots = 256 * t.per_cu, full = wgs / slots, rest = wgs % slots;
   const double step = full * t.full + (rest == 0 ? 0.0 : rest <= 256 ? t.one : t.full);
-  return 3.0 + (steps + 3) * step + (slices > 1 ? 4.0 + 2e-6 * slices * m * n : 0.0);
+  return 3.0 + (steps + 3.0) * step + (slices > 1 ? 4.0 + 2e-6 * slices * mn : 0.0);
 }
 
 }  // namespace
@@ -320,22 +320,29 @@ Gemm32Split gemm32_split(const bg_matmul_desc& d, bool wide, bool skinny, size_t
   Gemm32Split g;
   if (d.reserved == BG_MATMUL_F32_UNSPLIT) return g;
   if (skinny && !wide && d.m <= 32 && (!d.trans_b || d.n * d.k <= int64_t(10) << 20)) return g;
+  // The wide-K kernel's sizes, first without the model (a few hundred ns of the
+  // call): with up to 32 slices it says at least 9.1 us + k / 730, which is
+  // under 3 us + k / 128 only from k = 940 on.
+  if (wide && (d.m * d.n < 64 * 128 || d.k < 900)) return g;
   const int64_t as = ((d.m - 1) * d.lda + d.k) * 4;
   const int64_t bs = (d.trans_b ? (d.n - 1) * d.ldb + d.k : (d.k - 1) * d.ldb + d.n) * 4;
   if (as >= (int64_t(1) << 31) || bs >= (int64_t(1) << 31)) return g;
   double best = 0;
-  for (int c = 0; c < int(sizeof kTiles / sizeof kTiles[0]); ++c)
+  for (int c = 0; c < int(sizeof kTiles / sizeof kTiles[0]); ++c) {
+    const Tile& t = kTiles[c];
+    const int64_t tiles = (d.m + t.bm - 1) / t.bm * ((d.n + t.bn - 1) / t.bn) * d.batch;
     for (int s : {1, 2, 3, 4, 6, 8, 12, 16, 24, 32}) {
       if (s > 1 && (d.batch > 1 || d.k < 64 * s || s * d.m * d.n * 4 > kMaxPartials ||
                     size_t(s * d.m * d.n) * 4 + 256 > room))
         break;
-      const double t = model_us(kTiles[c], d.m, d.n, d.k, d.batch, s);
-      if (g.tile >= 0 && t >= best) continue;
-      best = t;
+      const double us = model_us(t, tiles, d.m * d.n, uint32_t(d.k), uint32_t(s));
+      if (g.tile >= 0 && us >= best) continue;
+      best = us;
       g.tile = c;
       g.slices = s;
     }
-  if (wide && (d.m * d.n < 64 * 128 || best > 3.0 + d.k / 128.0)) {
+  }
+  if (wide && best > 3.0 + d.k / 128.0) {
     g.tile = -1;
     return g;
   }
