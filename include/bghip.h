@@ -174,10 +174,12 @@ typedef struct bg_matmul_desc {
   int32_t reserved;      /* 0, or BG_MATMUL_F32_UNSPLIT */
 } bg_matmul_desc;
 
-/* An f32 product is taken from three bf16 parts of each operand (every f32
- * is their exact sum) on the bf16 matrix core, six partial products each,
- * with f32 sums: at least as close to the exact result as float32 products,
- * but the parts are signed, so sums of non-negative terms need not be
+/* An f32 product with K > 4 is taken from three bf16 parts of each operand
+ * (every f32 is their exact sum) on the bf16 matrix core: six of the nine
+ * partial products, with f32 sums.  What is left out is at most 2^-24 |a b|
+ * a term; the sums round less often, and the measured error against 64 bits
+ * (2-norm, and largest over sum |a b|) is below that of float32 products.
+ * The parts are signed, so sums of non-negative terms need not be
  * monotone.  With this value in `reserved` every product is formed by a
  * float32 matrix instruction (proofs that rest on monotone partial sums). */
 #define BG_MATMUL_F32_UNSPLIT 1

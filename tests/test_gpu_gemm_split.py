@@ -48,7 +48,7 @@ def _plan(m, n, k, trans_b):
 # and ragged tiles, K slices, K of one step and less, rows that allow no
 # 16-byte load, and a stage that K does not fill.
 SHAPES = [(4096, 4096, 64), (4001, 4003, 37), (2047, 3072, 100), (1500, 1500, 1500), (512, 1024, 768), (200, 2100, 515),
-          (65, 2200, 2049), (40, 3000, 700), (1, 9000, 500), (129, 65, 17), (300, 200, 1), (64, 128, 16)]
+          (65, 2200, 2049), (40, 3000, 700), (1, 9000, 500), (129, 65, 17), (300, 200, 5), (64, 128, 16)]
 
 
 @pytest.mark.parametrize("m,n,k", SHAPES)
@@ -75,6 +75,37 @@ def test_split_gemm_against_float64(bridge, m, n, k, trans_b):
     truth = a64 @ b64
     err = [np.linalg.norm(v - truth) / np.linalg.norm(truth) for v in (plain, unsplit)]
     assert err[0] <= 1.05 * err[1] + 2.0 ** -25, err
+
+
+@pytest.mark.parametrize("m,n", [(300, 200), (4096, 4096)])
+@pytest.mark.parametrize("k", [1, 2, 3, 4, 5, 6, 8])
+@pytest.mark.parametrize("near", [0.0, 1 + 2.0 ** -8])
+def test_few_terms_lose_no_precision(bridge, m, n, k, near):
+    """Random values, and mantissas near 1 + 2^-8, whose dropped part products are
+    largest (2^-24 of the product): K = 1 is the rounded product, up to K = 4 the
+    float32 kernel runs, and from K = 5 on no error (2-norm, largest over the mass)
+    is above the float32 kernel's."""
+    rng = np.random.default_rng(k)
+
+    def draw(*shape):
+        if near == 0.0:
+            return rng.standard_normal(shape).astype(F32)
+        x = F32(near) + F32(2.0 ** -23) * rng.integers(-64, 0, shape).astype(F32)
+        return x * rng.choice([-1, 1], shape).astype(F32)
+
+    a, b = draw(m, k), draw(k, n)
+    y, log = _gemm(bridge, a, b, False)
+    if k == 1:
+        assert np.array_equal(y, a * b)
+    if k <= 4:
+        assert "gemm32_kernel" in log[0]["kernel"]
+        return
+    assert "gemm32_split_kernel" in log[0]["kernel"]
+    unsplit, _ = _gemm(bridge, a, b, False, f32_unsplit=True)
+    a64, b64 = a.astype(np.float64), b.astype(np.float64)
+    truth, mass = a64 @ b64, np.abs(a64) @ np.abs(b64)
+    err = [(np.linalg.norm(v - truth), np.max(np.abs(v - truth) / mass)) for v in (y, unsplit)]
+    assert err[0][0] <= err[1][0] and err[0][1] <= err[1][1], err
 
 
 def test_split_gemm_batched(bridge):
