@@ -5,6 +5,7 @@ import ctypes as C
 
 import numpy as np
 import pytest
+import torch
 
 from browsergrad_amd import _native as N
 
@@ -153,7 +154,6 @@ def test_split_gemm_special_values(bridge, m, n, k, trans_b):
 def test_split_gemm_no_allocation(bridge):
     """Without workspace for the K slices the call takes fewer of them and
     still runs."""
-    import torch
     m, n, k = 1000, 4096, 4096
     a, b = torch.randn(m, k, device="cuda"), torch.randn(n, k, device="cuda")
     c = torch.zeros(m, n, device="cuda")
