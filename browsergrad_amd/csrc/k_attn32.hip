@@ -298,10 +298,12 @@ __global__ void __launch_bounds__(kNW * 64, 2) fa32_fwd_kernel(Fa32Args P) {
 // -> 60 us, B8 H16 S2048 causal 614 -> 462, one head of 2048 163 -> 92 (a
 // one-buffer form of four wavefronts, two workgroups a CU: 99 / 458 / 152).
 // Error against float64, 2-norm, B4 H12 S1000: 2.2e-7 (fa32_fwd_kernel 3.3e-7).
-// The parts hold values down to 2^-109 and finite ones; a workgroup that saw
-// others, or whose sums are not finite, redoes its queries one at a time in
-// float32 (fa32_plain).  Weights P below 2^-109 of their row's largest lose
-// bits: an error under 2^-133 max |v|.
+// Q, K, V and P are split times kSplitScale (Q's factor and the scores' 2^-48
+// cost nothing: they ride on the scale and on the subtraction of the maximum), so
+// no value and no weight that float32 holds loses bits.  (A maximum kept 24 lower,
+// which scales P for free, doubles the error: the exponents round at 24 instead
+// of at 1.)  A workgroup whose sums are not finite redoes its queries one at a
+// time in float32 (fa32_plain).
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 constexpr int kSplitNT = 512;  // wavefront w: queries 32 (w % 4) .., keys 32 (w / 4) .. of every tile
@@ -366,7 +368,7 @@ __global__ void __launch_bounds__(kSplitNT, 2) split_fa32_fwd_kernel(Fa32Args P,
   const float* Mp = P.mask ? P.mask + b * P.m_sb + h * P.m_sh : nullptr;
   const int nt_all = (P.Sk + kBK - 1) / kBK;
   const int nt = P.causal ? min(nt_all, (q0 + kBQ + kBK - 1) / kBK) : nt_all;
-  uint32_t low = bgk::kSplitTop;
+  const float q_scale = P.sl2 * bgk::kSplitScale;
 
   // B operand of the scores: Q[qi][16 c + 8 hi + j] * scale * log2(e).
   bgk::bf16x8 qf[NC][3];
@@ -377,10 +379,10 @@ __global__ void __launch_bounds__(kSplitNT, 2) split_fa32_fwd_kernel(Fa32Args P,
     for (int i = 0; i < 2; ++i) {
       const float4v v = load4<VEC>(Qp, P.q_ss, qi, P.Sq, 4 * c + 2 * hi + i, P.D);
 #pragma unroll
-      for (int j = 0; j < 4; ++j) x[4 * i + j] = v[j] * P.sl2;
+      for (int j = 0; j < 4; ++j) x[4 * i + j] = v[j] * q_scale;
     }
     u32x4 p1, p2, p3;
-    bgk::split8(x, p1, p2, p3, low);
+    bgk::split8(x, 1.f, p1, p2, p3);
     qf[c][0] = __builtin_bit_cast(bgk::bf16x8, p1);
     qf[c][1] = __builtin_bit_cast(bgk::bf16x8, p2);
     qf[c][2] = __builtin_bit_cast(bgk::bf16x8, p3);
@@ -443,7 +445,7 @@ __global__ void __launch_bounds__(kSplitNT, 2) split_fa32_fwd_kernel(Fa32Args P,
   };
   auto put = [&](u32x4* st, int plane, const float (&x)[8]) {
     u32x4 p1, p2, p3;
-    bgk::split8(x, p1, p2, p3, low);
+    bgk::split8(x, bgk::kSplitScale, p1, p2, p3);
     st[0] = p1;
     st[plane] = p2;
     st[2 * plane] = p3;
@@ -522,11 +524,11 @@ __global__ void __launch_bounds__(kSplitNT, 2) split_fa32_fwd_kernel(Fa32Args P,
     const int j0 = t * kBK + hh * 32;
     // A half wholly after the wavefront's queries, or past Sk, adds nothing.
     if (!(P.causal && j0 > q0w + kQW - 1) && j0 < P.Sk) {
-      // s[e]: key j0 + 8 (e / 4) + 4 hi + e % 4, query qi (log2 domain).
+      // s[e]: key j0 + 8 (e / 4) + 4 hi + e % 4, query qi (log2 domain, times 2^48).
       const bool edge = (P.causal && j0 + 31 > q0w) || j0 + 32 > P.Sk;
       if (Mp) {
 #pragma unroll
-        for (int e = 0; e < 16; ++e) s[e] = __builtin_fmaf(mv[e], kLog2e, s[e]);
+        for (int e = 0; e < 16; ++e) s[e] = __builtin_fmaf(mv[e], kLog2e / bgk::kSplitUnscale, s[e]);
       }
       if (edge) {
 #pragma unroll
@@ -539,7 +541,7 @@ __global__ void __launch_bounds__(kSplitNT, 2) split_fa32_fwd_kernel(Fa32Args P,
 #pragma unroll
       for (int e = 1; e < 16; ++e) mt = fmaxf(mt, s[e]);
       mt = fmaxf(mt, xor32(mt));
-      const float m_new = fmaxf(m_run, mt);
+      const float m_new = fmaxf(m_run, mt * bgk::kSplitUnscale);
       const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
       m_run = m_new;
       if (__builtin_amdgcn_ballot_w64(alpha != 1.0f)) {  // (NaN counts)
@@ -552,8 +554,8 @@ __global__ void __launch_bounds__(kSplitNT, 2) split_fa32_fwd_kernel(Fa32Args P,
       float l0 = 0.f, l1 = 0.f;
 #pragma unroll
       for (int e = 0; e < 16; e += 2) {
-        s[e] = __builtin_amdgcn_exp2f(s[e] - m_new);
-        s[e + 1] = __builtin_amdgcn_exp2f(s[e + 1] - m_new);
+        s[e] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[e], bgk::kSplitUnscale, -m_new));
+        s[e + 1] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[e + 1], bgk::kSplitUnscale, -m_new));
         l0 += s[e];
         l1 += s[e + 1];
       }
@@ -566,8 +568,7 @@ __global__ void __launch_bounds__(kSplitNT, 2) split_fa32_fwd_kernel(Fa32Args P,
 #pragma unroll
         for (int j = 0; j < 8; ++j) px[j] = s[8 * m + j];
         u32x4 pp[3];
-        uint32_t any = bgk::kSplitTop;
-        bgk::split8(px, pp[0], pp[1], pp[2], any);
+        bgk::split8(px, bgk::kSplitScale, pp[0], pp[1], pp[2]);
 #pragma unroll
         for (int db = 0; db < NDB; ++db) {
           bgk::bf16x8 vf[3];
@@ -597,7 +598,7 @@ __global__ void __launch_bounds__(kSplitNT, 2) split_fa32_fwd_kernel(Fa32Args P,
       for (int e = 0; e < 16; ++e) red[(2 + 16 * db + e) * 64] = acc[db][e];
   }
   __syncthreads();
-  bool redo = low < bgk::kSplitMin;
+  bool redo = false;
   if (hh == 0) {
     const float m = fmaxf(m_run, red[0]);
     const float f0 = __builtin_amdgcn_exp2f(m_run - m), f1 = __builtin_amdgcn_exp2f(red[0] - m);
@@ -612,9 +613,8 @@ __global__ void __launch_bounds__(kSplitNT, 2) split_fa32_fwd_kernel(Fa32Args P,
   }
   const int64_t ohead = int64_t(b) * P.o_sb + int64_t(h) * P.o_sh;
   const float lt = l_run + xor32(l_run);
-  const float inv = lt > 0.f ? 1.0f / lt : 0.f;
+  const float inv = lt > 0.f ? bgk::kSplitUnscale / lt : 0.f;
   redo |= hh == 0 && !(lt <= 3.402823466e38f);
-  // A value that the parts cannot hold may sit in a tile any thread staged.
   redo = __syncthreads_or(redo);
   if (hh == 1) return;
   if (redo) {

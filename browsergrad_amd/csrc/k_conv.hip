@@ -421,7 +421,6 @@ __global__ void __launch_bounds__(256, 2)
   const int b_d = int(kd) * P.dd - P.pd, b_h = int(kh) * P.dh - P.ph, b_w = int(kw) * P.dw - P.pw;
 
   float xa[8], xb[8];
-  uint32_t low = kSplitTop;
   // Byte offset of x's row for output row (n, od, oh), high bit set outside.
   auto x_row = [&](uint32_t n, uint32_t od, uint32_t oh, bool in) {
     const int id = int(od) * P.sd + b_d, ih = int(oh) * P.sh + b_h;
@@ -475,7 +474,7 @@ __global__ void __launch_bounds__(256, 2)
   };
   auto put = [&](u32x4* st, int plane, const float (&x)[8]) {
     u32x4 p1, p2, p3;
-    split8(x, p1, p2, p3, low);
+    split8(x, kSplitScale, p1, p2, p3);
     st[0] = p1;
     st[plane] = p2;
     st[2 * plane] = p3;
@@ -554,14 +553,17 @@ __global__ void __launch_bounds__(256, 2)
     slot = nslot;
   }
 
-  bool redo = low < kSplitMin;
+  bool redo = false;
 #pragma unroll
   for (int i = 0; i < TM; ++i)
 #pragma unroll
     for (int jt = 0; jt < TN; ++jt) {
       acc[i][jt] += small[i][jt];
 #pragma unroll
-      for (int e = 0; e < 16; ++e) redo |= !(fabsf(acc[i][jt][e]) <= 3.402823466e38f);
+      for (int e = 0; e < 16; ++e) {
+        redo |= !(fabsf(acc[i][jt][e]) <= 3.402823466e38f);
+        acc[i][jt][e] *= kSplitUnscale;
+      }
     }
   if (__syncthreads_or(redo)) {
 #pragma unroll

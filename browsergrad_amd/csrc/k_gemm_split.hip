@@ -75,7 +75,6 @@ __global__ void __launch_bounds__(64 * WGM * WGN, 2) gemm32_split_kernel(GemmArg
   }
 
   float xa[NA][8], xb[NB][8];
-  uint32_t low = kSplitTop;
   // Eight k of one row; lim: how many k of the stage lie before kend.
   auto load_row = [&](__amdgpu_buffer_rsrc_t rs, uint32_t off, int k0, int lim, float (&x)[8]) {
     if constexpr (ALIGNED) {
@@ -116,7 +115,7 @@ __global__ void __launch_bounds__(64 * WGM * WGN, 2) gemm32_split_kernel(GemmArg
   };
   auto put = [&](u32x4* st, int plane, const float (&x)[8]) {
     u32x4 p1, p2, p3;
-    split8(x, p1, p2, p3, low);
+    split8(x, kSplitScale, p1, p2, p3);
     st[0] = p1;
     st[plane] = p2;
     st[2 * plane] = p3;
@@ -212,22 +211,23 @@ __global__ void __launch_bounds__(64 * WGM * WGN, 2) gemm32_split_kernel(GemmArg
     slot = nslot;
   }
 
-  // Redo the tile in float32 where the split does not hold: a value too small
-  // for it, or an infinity, a NaN or an overflow (each leaves a sum that is
-  // not finite).
+  // Redo the tile in float32 where a sum is not finite.
   if constexpr (DUAL) {
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
       for (int j = 0; j < TN; ++j) acc[i][j] += small[i][j];
   }
-  bool redo = low < kSplitMin;
+  bool redo = false;
 #pragma unroll
   for (int i = 0; i < TM; ++i)
 #pragma unroll
     for (int j = 0; j < TN; ++j)
 #pragma unroll
-      for (int e = 0; e < 16; ++e) redo |= !(fabsf(acc[i][j][e]) <= 3.402823466e38f);
+      for (int e = 0; e < 16; ++e) {
+        redo |= !(fabsf(acc[i][j][e]) <= 3.402823466e38f);
+        acc[i][j][e] *= kSplitUnscale;
+      }
   if (__syncthreads_or(redo)) {
 #pragma unroll
     for (int i = 0; i < TM; ++i)

@@ -18,17 +18,20 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4s __attribute__((ext_vector_type(4)));
 
-// Smallest magnitude that splits exactly: the third part of x reaches down to
-// 2^-23 |x|, and bf16's smallest step is 2^-133.  split8 keeps the minimum of
-// 2 * magnitude bits - 2 over the nonzero values it sees (zero wraps to the
-// top); a kernel whose minimum is below kSplitMin redoes its tile in float32.
-constexpr uint32_t kSplitTop = 0xffffffffu;
-constexpr uint32_t kSplitMin = ((127u - 109u) << 24) - 2u;  // 2^-109
+// Operands are split times kSplitScale: the third part of x reaches down to
+// 2^-23 |x|, and the last place of any float32, 2^-149, becomes 2^-125, so that
+// every part of every finite value is a normal bf16 number.  A sum of products
+// comes out times kSplitScale^2.  (Unscaled, values below 2^-109, such as
+// softmax tails, cannot be held: kernels that redid their tiles for them took
+// 2 to 170 times as long with a single such value in an operand.)  Infinities,
+// NaN, values of 2^104 and more and results of 2^80 and more leave sums that are
+// not finite; such a tile is redone in float32.
+constexpr float kSplitScale = 16777216.f;                // 2^24
+constexpr float kSplitUnscale = 1.f / (16777216.f * 16777216.f);  // 2^-48
 
-// Splits two values into the packed bf16 parts.
-__device__ __forceinline__ void split2(float x0, float x1, uint32_t& p1, uint32_t& p2, uint32_t& p3, uint32_t& low) {
+// Splits two values, already times kSplitScale, into the packed bf16 parts.
+__device__ __forceinline__ void split2(float x0, float x1, uint32_t& p1, uint32_t& p2, uint32_t& p3) {
   const f32x2 v = {x0, x1};
-  low = min(low, min((__float_as_uint(x0) << 1) - 2u, (__float_as_uint(x1) << 1) - 2u));
   p1 = __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2));
   const f32x2 r = {x0 - __uint_as_float(p1 << 16), x1 - __uint_as_float(p1 & 0xffff0000u)};
   p2 = __builtin_bit_cast(uint32_t, __builtin_convertvector(r, bf16x2));
@@ -36,12 +39,12 @@ __device__ __forceinline__ void split2(float x0, float x1, uint32_t& p1, uint32_
   p3 = __builtin_bit_cast(uint32_t, __builtin_convertvector(q, bf16x2));
 }
 
-// Splits eight consecutive values.
-__device__ __forceinline__ void split8(const float (&x)[8], u32x4s& p1, u32x4s& p2, u32x4s& p3, uint32_t& low) {
+// Splits eight consecutive values times `scale` (1 or kSplitScale).
+__device__ __forceinline__ void split8(const float (&x)[8], float scale, u32x4s& p1, u32x4s& p2, u32x4s& p3) {
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     uint32_t a, b, c;
-    split2(x[2 * i], x[2 * i + 1], a, b, c, low);
+    split2(x[2 * i] * scale, x[2 * i + 1] * scale, a, b, c);
     p1[i] = a;
     p2[i] = b;
     p3[i] = c;

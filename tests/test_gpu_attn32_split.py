@@ -96,6 +96,49 @@ def test_split_attention_mask_and_views(bridge):
     assert np.all(np.abs(y.reshape(B, S, H, D).transpose(0, 2, 1, 3) - truth) <= 1e-5 * mass)
 
 
+@pytest.mark.parametrize("e", [-100, -115, -120])
+def test_split_attention_small_values(bridge, e):
+    """V, or K with Q scaled up, at 2^-100 to 2^-120: the bits of the unscaled
+    call, since such values take no other path."""
+    rng = np.random.default_rng(4)
+    b, h, s, d = 1, 2, 200, 64
+    q, k, v = (rng.uniform(1, 2, (b, h, s, d)).astype(F32) * rng.choice([-1, 1], (b, h, s, d)).astype(F32)
+               for _ in range(3))
+    kw = dict(batch=b, heads=h, sq=s, sk=s, d=d, scale=2.0 ** -4)
+
+    def run(*x):
+        hs = [bridge.upload(t, t.shape, "float32") for t in x]
+        y, log = _run(bridge, hs, **kw)
+        assert "split_fa32_fwd_kernel" in log[0]["kernel"]
+        for t in hs:
+            bridge.release(t)
+        return y.astype(np.float64)
+
+    base = run(q, k, v)
+    f = F32(2.0 ** e)
+    assert np.array_equal(run(q * F32(2.0 ** 60), k * f, v), run(q * F32(2.0 ** (60 + e)), k, v))
+    y = run(q, k, v * f)
+    normal = np.abs(y) >= 2.0 ** -126  # (below, the result itself rounds)
+    assert np.array_equal(y[normal], (base * 2.0 ** e)[normal]) and np.mean(normal) > 0.9
+
+
+def test_split_attention_small_weights(bridge):
+    """Weights of 2^-122 of the largest, whose key has V = 0, keep their bits: the
+    scores' roundings (122 * 2^-24, times ln 2) and a few units bound the error."""
+    s, d = 130, 64
+    rng = np.random.default_rng(6)
+    q, k = np.zeros((1, 1, 8, d), F32), np.zeros((1, 1, s, d), F32)
+    q[..., 0] = 1
+    k[0, 0, 1:, 0] = -122 * np.log(2) + rng.uniform(-1, 1, s - 1)
+    v = rng.uniform(1, 2, (1, 1, s, d)).astype(F32)
+    v[0, 0, 0] = 0
+    hs = [bridge.upload(t, t.shape, "float32") for t in (q, k, v)]
+    y, log = _run(bridge, hs, batch=1, heads=1, sq=8, sk=s, d=d, scale=1.0)
+    assert "split_fa32_fwd_kernel" in log[0]["kernel"]
+    truth, _ = _truth(q, k, v, 1.0, False)
+    assert np.all(np.abs(y - truth) <= (123 * 3 + 8) * 2.0 ** -24 * truth)
+
+
 @pytest.mark.parametrize("what", ["nan_k", "inf_v", "neg_inf_k", "tiny_v", "tiny_k", "huge_q"])
 def test_split_attention_special_values(bridge, what):
     """What the parts cannot hold gives what the float32 kernel gives."""

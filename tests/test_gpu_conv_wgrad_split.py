@@ -81,6 +81,20 @@ def test_weight_gradient_against_float64(bridge, n, c, o, size, kernel, stride, 
     assert (np.abs(got - want) <= 8 * np.sqrt(terms) * 2.0**-24 * mass + 1e-6).all()
 
 
+@pytest.mark.parametrize("e", [-100, -115, -126])
+@pytest.mark.parametrize("o", [40, 130])
+def test_small_values_take_no_other_path(bridge, e, o):
+    """dy at 2^-100 to 2^-126 against an x scaled up, and the other way round:
+    the unscaled gradient's bits."""
+    geo = ((3, 3), (1, 1), (1, 1), (1, 1))
+    x, dy = _data(2, 16, o, (10, 10), *geo, False, 5)
+    x, dy = (np.sign(t) * (F32(1) + np.abs(t) % F32(1)) for t in (x, dy))
+    base = _run(bridge, x, dy, *geo, 1, False).astype(np.float64)
+    lo, up = F32(2.0**e), F32(2.0**60)
+    for a, b in ((x * up, dy * lo), (x * lo, dy * up)):
+        assert np.array_equal(_run(bridge, a, b, *geo, 1, False).astype(np.float64), base * 2.0**(60 + e))
+
+
 @pytest.mark.parametrize("value", [2.0**-120, 1e-40, np.inf, np.nan, 3.4e38])
 def test_values_the_parts_cannot_hold(bridge, value):
     """A dy value below 2^-109, infinite, NaN or one whose leading part rounds to

@@ -151,6 +151,31 @@ def test_split_gemm_special_values(bridge, m, n, k, trans_b):
     assert np.all(np.abs(y[fin].astype(np.float64) - truth[fin]) <= bound)
 
 
+@pytest.mark.parametrize("e", [-100, -109, -115, -126, -135, -145])
+@pytest.mark.parametrize("m,n,k", [(70, 2100, 515), (300, 300, 40), (4096, 4096, 48)])
+def test_split_gemm_small_values(bridge, m, n, k, e):
+    """Full 24-bit mantissas down to float32's subnormals, against a B scaled up:
+    within the bound of float32 sums, element by element, and (where scaling loses
+    no bits) the unscaled product's very bits: such values take no other path."""
+    rng = np.random.default_rng(-e)
+    base = rng.uniform(1, 2, (m, k)).astype(F32) * rng.choice([-1, 1], (m, k)).astype(F32)
+    b = rng.standard_normal((k, n)).astype(F32)
+    a = (base.astype(np.float64) * 2.0 ** e).astype(F32)
+    up = b * F32(2.0 ** 60)
+    y, log = _gemm(bridge, a, up, False)
+    assert "gemm32_split_kernel" in log[0]["kernel"]
+    a64, b64 = a.astype(np.float64), up.astype(np.float64)
+    assert np.all(np.abs(y - a64 @ b64) <= 2.0 * np.sqrt(k) * 2.0 ** -24 * (np.abs(a64) @ np.abs(b64)))
+    if e >= -126:
+        plain, _ = _gemm(bridge, base, b, False)
+        assert np.array_equal(y.astype(np.float64), plain.astype(np.float64) * 2.0 ** (60 + e))
+    mixed = base.copy()
+    mixed[5, 3] = a[5, 3]  # one of them among ordinary values
+    y, _ = _gemm(bridge, mixed, b, False)
+    m64, b64 = mixed.astype(np.float64), b.astype(np.float64)
+    assert np.all(np.abs(y - m64 @ b64) <= 2.0 * np.sqrt(k) * 2.0 ** -24 * (np.abs(m64) @ np.abs(b64)))
+
+
 def test_split_gemm_no_allocation(bridge):
     """Without workspace for the K slices the call takes fewer of them and
     still runs."""
