@@ -111,16 +111,16 @@ __device__ __forceinline__ float4v load4(const float* base, int64_t ss, int row,
 }
 
 // DP: head dim rounded up to 16, 32 or 64 (the MFMA d loop covers DP / 2
-// values per half-wavefront; columns past D are zero in LDS and registers).
-template <int DP, bool VEC>
-__global__ void __launch_bounds__(kNW * 64, 2) fa32_fwd_kernel(Fa32Args P) {
+// values per half-wavefront; columns past D are zero in LDS and registers).  NT
+// threads stage; the first kNW wavefronts compute.
+// lds: two buffers of a K tile and a V tile, 64 rows x 256 bytes each.
+constexpr int kFa32Lds = 2 * 2 * kBK * 256;
+
+template <int DP, bool VEC, int NT>
+__device__ __forceinline__ void fa32_tiles(const Fa32Args& P, float* lds) {
   constexpr int NG = DP / 8;             // 16-byte K reads per lane per half (4 MFMAs each)
   constexpr int NDB = DP > 32 ? 2 : 1;   // 32-row blocks of O^T
   constexpr int CH = DP / 4;             // 16-byte chunks per row that hold data
-  // Two buffers of a K tile and a V tile, 64 rows x 256 bytes each.
-  __shared__ float4v smem[2 * 2 * kBK * 16];
-  float* lds = reinterpret_cast<float*>(smem);
-
   const int lane = threadIdx.x & 63;
   const int w = threadIdx.x >> 6;
   const int hi = lane >> 5;
@@ -149,14 +149,14 @@ __global__ void __launch_bounds__(kNW * 64, 2) fa32_fwd_kernel(Fa32Args P) {
     for (int i = 0; i < 4; ++i) qf[g][i] = x[i] * P.sl2;
   }
 
-  // Tile staging: thread t moves 16-byte units t, t + 256, ... of the K and
+  // Tile staging: thread t moves 16-byte units t, t + NT, ... of the K and
   // V tiles (unit u = row u / 16, chunk u % 16; chunks past DP / 4 stay 0).
-  constexpr int UNITS = kBK * 16 / (kNW * 64);  // 4
+  constexpr int UNITS = kBK * 16 / NT;
   float4v kst[UNITS], vst[UNITS];
   auto fetch = [&](int t) {
 #pragma unroll
     for (int s = 0; s < UNITS; ++s) {
-      const int u = threadIdx.x + s * kNW * 64;
+      const int u = threadIdx.x + s * NT;
       const int row = u >> 4, c = u & 15;
       const int key = t * kBK + row;
       kst[s] = c < CH ? load4<VEC>(Kp, P.k_ss, key, P.Sk, c, P.D) : float4v{0.f, 0.f, 0.f, 0.f};
@@ -168,7 +168,7 @@ __global__ void __launch_bounds__(kNW * 64, 2) fa32_fwd_kernel(Fa32Args P) {
     float* vt = kt + kBK * 64;
 #pragma unroll
     for (int s = 0; s < UNITS; ++s) {
-      const int u = threadIdx.x + s * kNW * 64;
+      const int u = threadIdx.x + s * NT;
       const int row = u >> 4, c = u & 15;
       *reinterpret_cast<float4v*>(kt + k_slot(row, c)) = kst[s];
       *reinterpret_cast<float4v*>(vt + v_slot(row, c)) = vst[s];
@@ -195,6 +195,7 @@ __global__ void __launch_bounds__(kNW * 64, 2) fa32_fwd_kernel(Fa32Args P) {
 #pragma unroll
     for (int hh = 0; hh < 2; ++hh) {
       const int j0 = t * kBK + hh * 32;
+      if (NT > kNW * 64 && w >= kNW) continue;
       // A half wholly after the wavefront's last query adds nothing (causal).
       if (P.causal && j0 > q0w + kQW - 1) continue;
       if (j0 >= P.Sk) continue;
@@ -267,7 +268,7 @@ __global__ void __launch_bounds__(kNW * 64, 2) fa32_fwd_kernel(Fa32Args P) {
   // O^T[d = 32 db + 8 (e / 4) + 4 hi + e % 4][qi].
   const float lt = l_run + xor32(l_run);
   const float inv = lt > 0.f ? 1.0f / lt : 0.f;
-  if (qi >= P.Sq) return;
+  if (qi >= P.Sq || (NT > kNW * 64 && w >= kNW)) return;
   const int64_t obase = int64_t(b) * P.o_sb + int64_t(h) * P.o_sh + int64_t(qi) * P.o_ss;
 #pragma unroll
   for (int db = 0; db < NDB; ++db)
@@ -276,6 +277,12 @@ __global__ void __launch_bounds__(kNW * 64, 2) fa32_fwd_kernel(Fa32Args P) {
       const int d = 32 * db + 8 * (e >> 2) + 4 * hi + (e & 3);
       if (d < P.D) bgk::store_from_f32(P.o, P.out_dtype, obase + d, acc[db][e] * inv);
     }
+}
+
+template <int DP, bool VEC>
+__global__ void __launch_bounds__(kNW * 64, 2) fa32_fwd_kernel(Fa32Args P) {
+  __shared__ float4v smem[kFa32Lds / 16];
+  fa32_tiles<DP, VEC, kNW * 64>(P, reinterpret_cast<float*>(smem));
 }
 
 // ---- the same attention on the bf16 matrix core ------------------------------------
@@ -302,46 +309,11 @@ __global__ void __launch_bounds__(kNW * 64, 2) fa32_fwd_kernel(Fa32Args P) {
 // cost nothing: they ride on the scale and on the subtraction of the maximum), so
 // no value and no weight that float32 holds loses bits.  (A maximum kept 24 lower,
 // which scales P for free, doubles the error: the exponents round at 24 instead
-// of at 1.)  A workgroup whose sums are not finite redoes its queries one at a
-// time in float32 (fa32_plain).
+// of at 1.)  A workgroup whose sums are not finite redoes its queries in
+// float32 as fa32_fwd_kernel does (fa32_tiles), with its bits.
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 constexpr int kSplitNT = 512;  // wavefront w: queries 32 (w % 4) .., keys 32 (w / 4) .. of every tile
-
-// Queries q0w .. +31 of one wavefront in float32: one key per lane for the
-// scores, one output column per lane for P V.
-__device__ __forceinline__ void fa32_plain(const Fa32Args& P, const float* Qp, const float* Kp,
-                                                     const float* Vp, const float* Mp, int64_t ohead, int q0w) {
-  const int lane = threadIdx.x & 63;
-  const bool col = lane < P.D;
-  for (int qi = q0w; qi < min(q0w + kQW, P.Sq); ++qi) {
-    const int keys = P.causal ? min(P.Sk, qi + 1) : P.Sk;
-    const float* qr = Qp + int64_t(qi) * P.q_ss;
-    float m = kMSentinel, l = 0.f, o = 0.f;
-    for (int j0 = 0; j0 < keys; j0 += 64) {
-      const int j = j0 + lane;
-      float s = -INFINITY;
-      if (j < keys) {
-        s = 0.f;
-        for (int d = 0; d < P.D; ++d) s = __builtin_fmaf(qr[d] * P.sl2, Kp[int64_t(j) * P.k_ss + d], s);
-        if (Mp) s = __builtin_fmaf(Mp[int64_t(qi) * P.m_ss + j], kLog2e, s);
-      }
-      float mt = s;
-      for (int x = 1; x < 64; x <<= 1) mt = fmaxf(mt, __shfl_xor(mt, x));
-      const float m_new = fmaxf(m, mt), alpha = __builtin_amdgcn_exp2f(m - m_new);
-      m = m_new;
-      const float p = __builtin_amdgcn_exp2f(s - m_new);
-      l = l * alpha + bgk::wave_sum(p);
-      o *= alpha;
-      for (int x = 0; x < min(64, keys - j0); ++x) {
-        const float px = __shfl(p, x);
-        if (col) o = __builtin_fmaf(px, Vp[int64_t(j0 + x) * P.v_ss + lane], o);
-      }
-    }
-    if (col)
-      bgk::store_from_f32(P.o, P.out_dtype, ohead + int64_t(qi) * P.o_ss + lane, l > 0.f ? o * (1.0f / l) : l == l ? 0.f : l);
-  }
-}
 
 template <int DP, bool VEC>
 __global__ void __launch_bounds__(kSplitNT, 2) split_fa32_fwd_kernel(Fa32Args P, uint32_t k_bytes,
@@ -352,7 +324,9 @@ __global__ void __launch_bounds__(kSplitNT, 2) split_fa32_fwd_kernel(Fa32Args P,
   constexpr int VU = 4 * NDB * 64;       // 32 NDB columns x 8 sets of eight keys
   constexpr int NK = (KU + kSplitNT - 1) / kSplitNT, NV = (VU + kSplitNT - 1) / kSplitNT;
   constexpr int BUF = 3 * (KU + VU);
-  __shared__ u32x4 smem[2 * BUF > 4 * 64 * 9 ? 2 * BUF : 4 * 64 * 9];
+  // (4 * 64 * 9 units hold the halves' merge, kFa32Lds bytes the float32 redo.)
+  static_assert(kFa32Lds / 16 >= 4 * 64 * 9, "the redo's buffers cover the merge");
+  __shared__ u32x4 smem[2 * BUF > kFa32Lds / 16 ? 2 * BUF : kFa32Lds / 16];
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -616,12 +590,11 @@ __global__ void __launch_bounds__(kSplitNT, 2) split_fa32_fwd_kernel(Fa32Args P,
   const float inv = lt > 0.f ? bgk::kSplitUnscale / lt : 0.f;
   redo |= hh == 0 && !(lt <= 3.402823466e38f);
   redo = __syncthreads_or(redo);
-  if (hh == 1) return;
   if (redo) {
-    fa32_plain(P, Qp, Kp, Vp, Mp, ohead, q0w);
+    fa32_tiles<DP, VEC, kSplitNT>(P, reinterpret_cast<float*>(smem));
     return;
   }
-  if (qi >= P.Sq) return;
+  if (hh == 1 || qi >= P.Sq) return;
 #pragma unroll
   for (int db = 0; db < NDB; ++db)
 #pragma unroll
@@ -750,10 +723,10 @@ void plan_attention(const bg_attention_desc& d0, bg_launch_plan& out) {
   out.tile_n = kBK;
   out.tile_k = dp;
   out.k_slices = 1;
-  out.lds_bytes = 2 * 2 * kBK * 16 * 16;
+  out.lds_bytes = kFa32Lds;
   out.n_launches = 1;
   const bool split = fa32_split(d);
-  if (split) out.lds_bytes = std::max(2 * 3 * 16 * (dp * 8 + (dp > 32 ? 512 : 256)), 4 * 64 * 9 * 16);
+  if (split) out.lds_bytes = std::max(2 * 3 * 16 * (dp * 8 + (dp > 32 ? 512 : 256)), kFa32Lds);
   bg_launch_plan_entry& e = out.launch[0];
   std::snprintf(e.family, sizeof e.family, "%s", split ? "split_fa32_fwd_kernel" : "fa32_fwd_kernel");
   e.n_targs = 2;

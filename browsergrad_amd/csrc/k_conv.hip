@@ -572,34 +572,20 @@ __global__ void __launch_bounds__(256, 2)
       for (int jt = 0; jt < TN; ++jt)
 #pragma unroll
         for (int e = 0; e < 16; ++e) acc[i][jt][e] = 0.f;
-    for (int k = kbeg; k < kend; k += 2) {  // float32 MFMAs: k = lane / 32 on both operands
-      const bool k_ok = k + (lane >> 5) < kend;
-      const uint32_t ke = k_ok ? uint32_t(k + (lane >> 5)) : 0u;
-      const uint32_t n = fdiv(ke, P.f_oS), sp = ke - n * uint32_t(P.oS);
-      const uint32_t od = fdiv(sp, P.f_oHW), r = sp - od * uint32_t(oHW);
-      const uint32_t oh = fdiv(r, P.f_oW), ow = r - oh * uint32_t(P.oW);
-      float b[TN];
+    // The same stages, as float32 in k-major rows of two LDS buffers.
+    constexpr int LA = BM + 4, LB = BN + 4;
+    load_stage(0);
+    for (int t = 0; t < nk; ++t) {
+      float* as = reinterpret_cast<float*>(smem) + (t & 1) * 16 * (LA + LB);
+      float* bs = as + 16 * LA;
 #pragma unroll
-      for (int jt = 0; jt < TN; ++jt) {
-        const int col = n0 + wn * (BN / WGN) + jt * 32 + (lane & 31);
-        const uint32_t cc = col < P.NC ? uint32_t(col) : 0u;
-        const uint32_t ch = fdiv(cc, P.f_KV), v = cc - ch * uint32_t(P.KV);
-        const uint32_t vd = fdiv(v, P.f_KHW), vr = v - vd * uint32_t(KHW);
-        const uint32_t vh = fdiv(vr, P.f_KW), vw = vr - vh * uint32_t(P.KW);
-        const int id = int(od) * P.sd + int(vd) * P.dd - P.pd, ih = int(oh) * P.sh + int(vh) * P.dh - P.ph,
-                  iw = int(ow) * P.sw + int(vw) * P.dw - P.pw;
-        const bool ok = k_ok && col < P.NC && unsigned(id) < unsigned(P.D) && unsigned(ih) < unsigned(P.H) &&
-                        unsigned(iw) < unsigned(P.W);
-        b[jt] = ok ? P.b[(int64_t(n) * P.C + g * P.Cpg + ch) * P.S + (int64_t(id) * P.H + ih) * P.W + iw] : 0.f;
+      for (int e = 0; e < 8; ++e) {
+        if (UA >= NT || wave * 64 < UA) as[(8 * ac + e) * LA + ar] = xa[e];
+        bs[(8 * bk + e) * LB + bc] = xb[e];
       }
-#pragma unroll
-      for (int i = 0; i < TM; ++i) {
-        const int row = m0 + wm * (BM / WGM) + i * 32 + (lane & 31);
-        const float a = k_ok && row < P.M ? P.a[(int64_t(n) * P.O + g * P.Opg + row) * P.oS + sp] : 0.f;
-#pragma unroll
-        for (int jt = 0; jt < TN; ++jt)
-          acc[i][jt] = __builtin_amdgcn_mfma_f32_32x32x2f32(a, b[jt], acc[i][jt], 0, 0, 0);
-      }
+      __syncthreads();
+      load_stage(t + 1);
+      mul_stage_f32<LA, LB>(as + wm * (BM / WGM), bs + wn * (BN / WGN), acc);
     }
   }
 #pragma unroll

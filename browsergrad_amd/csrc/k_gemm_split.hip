@@ -235,25 +235,30 @@ __global__ void __launch_bounds__(64 * WGM * WGN, 2) gemm32_split_kernel(GemmArg
       for (int j = 0; j < TN; ++j)
 #pragma unroll
         for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
-    // MFMA q of an 8-deep step takes k = 4 (lane / 32) + q on both operands.
-    for (int k = kbeg; k < kend; k += 8) {
+    // The same stages, as float32 in k-major rows of two LDS buffers.
+    constexpr int LA = BM + 4, LB = BN + 4;
+    load_stage(0);
+    for (int t = 0; t < nk; ++t) {
+      float* as = reinterpret_cast<float*>(smem) + (t & 1) * 16 * (LA + LB);
+      float* bs = as + 16 * LA;
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const int64_t kk = k + 4 * (lane >> 5) + q;
-        float b[TN];
+      for (int i = 0; i < NA; ++i) {
+        const int u = i * NT + tid;
 #pragma unroll
-        for (int j = 0; j < TN; ++j) {
-          const int64_t n = n0 + wn * WTN + j * 32 + (lane & 31);
-          b[j] = kk < kend && n < P.N ? (TRANS_B ? B[n * P.ldb + kk] : B[kk * P.ldb + n]) : 0.f;
-        }
-#pragma unroll
-        for (int i = 0; i < TM; ++i) {
-          const int64_t m = m0 + wm * WTM + i * 32 + (lane & 31);
-          const float a = kk < kend && m < P.M ? A[m * P.lda + kk] : 0.f;
-#pragma unroll
-          for (int j = 0; j < TN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a, b[j], acc[i][j], 0, 0, 0);
-        }
+        for (int j = 0; j < 8; ++j)
+          if (UA % NT == 0 || i * NT + wave * 64 < UA) as[(8 * (u & 1) + j) * LA + (u >> 1)] = xa[i][j];
       }
+#pragma unroll
+      for (int i = 0; i < NB; ++i) {
+        const int u = i * NT + tid;
+        const int r = TRANS_B ? u >> 1 : u % BN, c = TRANS_B ? u & 1 : u / BN;
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+          if (UB % NT == 0 || i * NT + wave * 64 < UB) bs[(8 * c + j) * LB + r] = xb[i][j];
+      }
+      __syncthreads();
+      if (t + 1 < nk) load_stage(t + 1);
+      mul_stage_f32<LA, LB>(as + wm * WTM, bs + wn * WTN, acc);
     }
   }
 

@@ -51,4 +51,23 @@ __device__ __forceinline__ void split8(const float (&x)[8], float scale, u32x4s&
   }
 }
 
+// The float32 redo: one 16-deep stage of float32 MFMAs from k-major LDS rows
+// (LA and LB floats long; as and bs at the wavefront's first row and column).
+template <int LA, int LB, int TM, int TN, typename Acc>
+__device__ __forceinline__ void mul_stage_f32(const float* as, const float* bs, Acc (&acc)[TM][TN]) {
+  const int l32 = threadIdx.x & 31, hi = (threadIdx.x >> 5) & 1;
+#pragma unroll
+  for (int q = 0; q < 8; ++q) {
+    float a[TM], b[TN];
+#pragma unroll
+    for (int i = 0; i < TM; ++i) a[i] = as[(2 * q + hi) * LA + i * 32 + l32];
+#pragma unroll
+    for (int j = 0; j < TN; ++j) b[j] = bs[(2 * q + hi) * LB + j * 32 + l32];
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i], b[j], acc[i][j], 0, 0, 0);
+  }
+}
+
 }  // namespace bgk

@@ -96,6 +96,25 @@ def test_split_attention_mask_and_views(bridge):
     assert np.all(np.abs(y.reshape(B, S, H, D).transpose(0, 2, 1, 3) - truth) <= 1e-5 * mass)
 
 
+@pytest.mark.parametrize("d", [7, 16, 32, 33, 64])
+@pytest.mark.parametrize("causal", [False, True])
+def test_redo_is_the_float32_kernel(bridge, d, causal):
+    """A workgroup that met a NaN gives the float32 kernel's bits, every padded
+    head dim and both kinds of load; the other head does not notice."""
+    rng = np.random.default_rng(d)
+    b, h, s = 1, 2, 300
+    q, k, v = (rng.standard_normal((b, h, s, d)).astype(F32) for _ in range(3))
+    kw = dict(batch=b, heads=h, sq=s, sk=s, d=d, scale=d ** -0.5, causal=causal)
+    hs = [bridge.upload(t, t.shape, "float32") for t in (q, k, v)]
+    clean, _ = _run(bridge, hs, **kw)
+    v[0, 0, 0, d - 1] = np.nan  # every query of the head sees it
+    hs[2] = bridge.upload(v, v.shape, "float32")
+    y, log = _run(bridge, hs, **kw)
+    t, _ = _run(bridge, hs, tiled=True, **kw)
+    assert "split_fa32_fwd_kernel" in log[0]["kernel"] and np.isnan(t[0, 0, :, d - 1]).all()
+    assert np.array_equal(y[0, 0], t[0, 0], equal_nan=True) and np.array_equal(y[0, 1], clean[0, 1])
+
+
 @pytest.mark.parametrize("e", [-100, -115, -120])
 def test_split_attention_small_values(bridge, e):
     """V, or K with Q scaled up, at 2^-100 to 2^-120: the bits of the unscaled

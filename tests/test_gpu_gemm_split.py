@@ -151,6 +151,25 @@ def test_split_gemm_special_values(bridge, m, n, k, trans_b):
     assert np.all(np.abs(y[fin].astype(np.float64) - truth[fin]) <= bound)
 
 
+@pytest.mark.parametrize("m,n,k", [(300, 300, 40), (1001, 1003, 37), (2048, 1027, 64), (4096, 4096, 48)])
+@pytest.mark.parametrize("trans_b", [False, True])
+def test_redo_is_the_float32_kernel(bridge, m, n, k, trans_b):
+    """A tile that met a NaN gives the float32 kernel's bits (the same order of
+    sums); tiles that did not keep theirs."""
+    rng = np.random.default_rng(m)
+    a = rng.standard_normal((m, k)).astype(F32)
+    b = rng.standard_normal((n, k) if trans_b else (k, n)).astype(F32)
+    clean, _ = _gemm(bridge, a, b, trans_b)
+    a[m - 1, k - 1] = np.nan
+    y, log = _gemm(bridge, a, b, trans_b)
+    unsplit, other = _gemm(bridge, a, b, trans_b, f32_unsplit=True)
+    assert "gemm32_split_kernel" in log[0]["kernel"] and "gemm32_kernel" in other[0]["kernel"]
+    tile = _plan(m, n, k, trans_b)["tile"][0]
+    first = (m - 1) // tile * tile
+    assert np.array_equal(y[first:], unsplit[first:], equal_nan=True) and np.isnan(y[m - 1]).all()
+    assert np.array_equal(y[:first], clean[:first])
+
+
 @pytest.mark.parametrize("e", [-100, -109, -115, -126, -135, -145])
 @pytest.mark.parametrize("m,n,k", [(70, 2100, 515), (300, 300, 40), (4096, 4096, 48)])
 def test_split_gemm_small_values(bridge, m, n, k, e):
