@@ -525,6 +525,7 @@ __global__ void __launch_bounds__(256, 2)
   // t - 1 is free for stage t + 2 and stage t + 1 may be read.
   int slot = 0;
   for (int t = 0; t < nk; ++t) {
+    const bool more = BM < 128 || t + 2 < nk;
     const int nslot = slot == 2 ? 0 : slot + 1, wslot = slot == 0 ? 2 : slot - 1;
 #pragma unroll
     for (int i = 0; i < TM; ++i) {
@@ -543,10 +544,14 @@ __global__ void __launch_bounds__(256, 2)
       if (i == 0) {
         __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
         __builtin_amdgcn_s_barrier();
-        put_a(wslot);
+        // (With four tiles a wavefront the branch keeps the split behind the barrier:
+        // its first multiplies, moved before it, wait for the stage's loads, 1 x 256 x
+        // 64 x 64 with 256 filters 58.1 -> 54.6 us.  With two they wait less than the
+        // lost overlap costs: 32 x 64 x 56 x 56 107.0, with the branch 114.7.)
+        if (more) put_a(wslot);
       }
       if (i == 1) {
-        put_b(wslot);
+        if (more) put_b(wslot);
         load_stage(t + 3);
       }
     }
