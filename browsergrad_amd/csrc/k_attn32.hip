@@ -622,10 +622,21 @@ bool fa32_supported(const bg_attention_desc& d) {
 }
 
 // The split kernel from two key tiles on (one tile: 16 queries and keys 10.2
-// against 8.7 us, 64: 11.5 against 11.3); K and V of a head within a 32-bit
-// buffer offset.
+// against 8.7 us, 64: 11.5 against 11.3), and where it needs more than one round
+// of 256 workgroups (one a CU; the float32 kernel has two) only with more than
+// three key tiles for a query block on average: first loads, merge and
+// the uneven round cost more than the products save on few.  D64, split
+// against float32 kernel: 256 heads of 128 queries and keys 17 against 19 us, 384
+// heads 33 / 29, 1024 heads 67 / 60; 1024 heads of 8 queries and 128 keys 52 / 47,
+// 192 keys 62 / 65, 256 keys 73 / 82; causal, 1024 heads of 256 155 / 139, of 320
+// 239 / 238, of 512 395 / 411.  K and V of a head within a 32-bit buffer offset.
 static bool fa32_split(const bg_attention_desc& d) {
   const int64_t lim = int64_t(1) << 31;
+  const int64_t blocks = (d.sq + kBQ - 1) / kBQ, tiles = (d.sk + kBK - 1) / kBK;
+  if (d.batch * d.heads * blocks > 256) {
+    const int64_t cut = d.causal ? std::min(blocks, tiles / 2) : 0;  // block i sees 2 i + 2 tiles
+    if (cut * (cut + 1) + (blocks - cut) * tiles <= 3 * blocks) return false;
+  }
   return d.reserved != BG_ATTENTION_TILED && d.sk > kBK && ((d.sk - 1) * d.k_ss + d.d) * 4 < lim &&
          ((d.sk - 1) * d.v_ss + d.d) * 4 < lim && (d.sk + 2 * kBK) * d.k_ss * 4 < 2 * lim &&
          (d.sk + 2 * kBK) * d.v_ss * 4 < 2 * lim;

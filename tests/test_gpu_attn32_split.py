@@ -69,6 +69,29 @@ def test_split_attention(bridge, b, h, sq, sk, d, causal):
         bridge.release(x)
 
 
+# One round of 256 workgroups, one workgroup more with few and with more than
+# three key tiles a query block, and causal averages of 3 and 11 / 3 tiles.
+@pytest.mark.parametrize("h,sq,sk,causal,family", [
+    (256, 128, 128, False, "split_fa32_fwd_kernel"), (257, 128, 128, False, "fa32_fwd_kernel"),
+    (260, 8, 192, False, "fa32_fwd_kernel"), (260, 8, 193, False, "split_fa32_fwd_kernel"),
+    (130, 256, 256, True, "fa32_fwd_kernel"), (130, 320, 320, True, "split_fa32_fwd_kernel")])
+def test_kernel_choice(bridge, h, sq, sk, causal, family):
+    d = 8
+    rng = np.random.default_rng(h + sk)
+    q, k, v = (rng.standard_normal((1, h, n, d)).astype(F32) for n in (sq, sk, sk))
+    hs = [bridge.upload(t, t.shape, "float32") for t in (q, k, v)]
+    y, log = _run(bridge, hs, batch=1, heads=h, sq=sq, sk=sk, d=d, scale=d ** -0.5, causal=causal)
+    from browsergrad_amd.semantic import launch_plan
+    a = N.AttentionDesc()
+    a.batch, a.heads, a.sq, a.sk, a.d, a.causal = 1, h, sq, sk, d, int(causal)
+    a.in_dtype = a.out_dtype = N.BG_F32
+    plan = launch_plan("attention", a)["launches"]
+    assert plan[0]["family"] == family and f"{len(family)}{family}" in log[0]["kernel"]
+    assert [(r["grid"], r["block"]) for r in log] == [(e["grid"], e["block"]) for e in plan]
+    truth, mass = _truth(q, k, v, d ** -0.5, causal)
+    assert np.all(np.abs(y - truth) <= (4e-6 + 2.0 * np.sqrt(sk) * 2.0 ** -24) * mass)
+
+
 def test_split_attention_mask_and_views(bridge):
     """An additive mask (with a row of -inf, which gives zeros) and Q, K, V as
     views of one projection with an odd head dim."""
