@@ -202,16 +202,26 @@ void log_launch(bg_ctx* ctx, const void* kernel, dim3 grid, dim3 block, size_t s
 }
 
 void* scratch(bg_ctx* ctx, size_t bytes, int slot) {
-  if (bytes <= ctx->scratch_bytes[slot]) return ctx->scratch[slot];
+  const bool captured = ctx->scratch_captured[slot];
+  if (bytes <= ctx->scratch_bytes[slot]) {
+    if (!captured) ctx->scratch_captured[slot] = stream_capturing(ctx);
+    return ctx->scratch[slot];
+  }
   if (ctx->scratch[slot]) {
-    hip_check(hipStreamSynchronize(ctx->stream), "synchronize before scratch grow");
-    hip_check(hipFree(ctx->scratch[slot]), "hipFree(scratch)");
+    if (captured) {
+      ctx->captured_scratch.push_back(ctx->scratch[slot]);
+    } else {
+      hip_check(hipStreamSynchronize(ctx->stream), "synchronize before scratch grow");
+      hip_check(hipFree(ctx->scratch[slot]), "hipFree(scratch)");
+    }
     ctx->scratch[slot] = nullptr;
     ctx->scratch_bytes[slot] = 0;
+    ctx->scratch_captured[slot] = false;
   }
   size_t cap = pooled_size(bytes);
   hip_check(hipMalloc(&ctx->scratch[slot], cap), "hipMalloc(scratch)");
   ctx->scratch_bytes[slot] = cap;
+  ctx->scratch_captured[slot] = stream_capturing(ctx);
   return ctx->scratch[slot];
 }
 
@@ -368,6 +378,7 @@ int bg_ctx_destroy(bg_ctx* ctx) {
   for (auto e : ctx->event_pool) (void)hipEventDestroy(e);
   for (void* sp : ctx->scratch)
     if (sp) (void)hipFree(sp);
+  for (void* sp : ctx->captured_scratch) (void)hipFree(sp);
   (void)hipStreamDestroy(ctx->stream);
   delete ctx;
   return BG_OK;

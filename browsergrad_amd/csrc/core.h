@@ -87,13 +87,15 @@ struct bg_ctx {
   std::vector<hipEvent_t> event_pool;
   bg::Profile* active_profile = nullptr;
 
-  // Scratch buffers reused across launches (workspace for pre-passes):
-  // slot 0 = re-laid-out GEMM operand, slot 1 = f32 GEMM result awaiting an
-  // elementwise epilogue pass.
-  // GEMM scratch slots: 0 B re-layout / B cast, 1 f32 pre-GELU product,
-  // 2 A cast, 3 split-K partials.
+  // Scratch buffers reused across launches (workspace for pre-passes).  GEMM
+  // slots: 0 B re-layout / B cast, 1 f32 pre-GELU product, 2 A cast, 3 K-slice
+  // partials (and decode attention's key-slice partials).
   void* scratch[4] = {nullptr, nullptr, nullptr, nullptr};
   size_t scratch_bytes[4] = {0, 0, 0, 0};
+  // A buffer that a captured call used is named by a graph: when its slot grows
+  // it is kept here until the context ends instead of being freed.
+  bool scratch_captured[4] = {false, false, false, false};
+  std::vector<void*> captured_scratch;
 
   // Device address of this device's fixed no-allocation scratch (NULL when
   // it could not be resolved; bg_matmul_noalloc then refuses).
@@ -116,9 +118,9 @@ bg_handle mint_view(bg_ctx* ctx, const Record& src, int64_t offset,
                     int64_t nbytes, const std::vector<int64_t>& shape,
                     int dtype);
 void* scratch(bg_ctx* ctx, size_t bytes, int slot = 0);
-// True while the context's stream is captured into a graph: a later call may
-// grow (free) a scratch slot that the graph still names, so a call that can
-// do without partials then takes one slice.
+// True while the context's stream is captured into a graph.  A split GEMM or
+// decode attention then takes one slice, so that its graph holds one launch and
+// no scratch.
 bool stream_capturing(bg_ctx* ctx);
 std::vector<int64_t> to_shape(const int64_t* shape, int rank);
 int64_t numel(const std::vector<int64_t>& shape);

@@ -1,6 +1,5 @@
-"""Calls on a captured stream: what takes partial sums from the context's scratch
-outside a capture runs in one slice inside it, so that a replay does not
-depend on scratch that a later call may grow."""
+"""Calls on a captured stream: split GEMMs and decode attention run in one slice,
+and scratch that a graph names outlives the growth of its slot."""
 import numpy as np
 import pytest
 import torch
@@ -59,3 +58,61 @@ def test_captured_call_takes_no_scratch(bridge, make):
         br.release(fn())
         br.synchronize()
     br.release(h)
+
+
+def _skinny(br, rng, m, n, k, dtype):
+    a, b = rng.standard_normal((m, k)), rng.standard_normal((k, n))
+    if dtype == "float16":
+        a, b = a.astype(np.float16), np.ascontiguousarray(b.T.astype(np.float16))
+    else:
+        a, b = a.astype(F32), b.astype(F32)
+    ha, hb = br.upload(a, a.shape, dtype), br.upload(b, b.shape, dtype)
+    return lambda: br.matmul_ex(ha, hb, m=m, n=n, k=k, trans_b=dtype == "float16", in_dtype=dtype,
+                                out_dtype="float32")
+
+
+def _transposed_b(br, rng, n):
+    a, b = rng.standard_normal((96, 512)).astype(np.float16), rng.standard_normal((512, n)).astype(np.float16)
+    ha, hb = br.upload(a, a.shape, "float16"), br.upload(b, b.shape, "float16")
+    return lambda: br.matmul_ex(ha, hb, m=96, n=n, k=512, in_dtype="float16", out_dtype="float32")
+
+
+def _conv(br, rng, c):
+    x, dy = rng.standard_normal((2, c, 28, 28)).astype(F32), rng.standard_normal((2, 64, 28, 28)).astype(F32)
+    hx, hd = br.upload(x, x.shape, "float32"), br.upload(dy, dy.shape, "float32")
+    return lambda: br.conv_ex("backward_weight", hd, hx, n=2, c_in=c, c_out=64, in_size=(28, 28), out_size=(28, 28),
+                              k=(3, 3), stride=(1, 1), pad=(1, 1), dilation=(1, 1))
+
+
+# A call that keeps something in scratch, and a larger one in the same slot.
+@pytest.mark.parametrize("small,large", [
+    (lambda br, g: _skinny(br, g, 1, 4096, 4096, "float32"), lambda br, g: _skinny(br, g, 64, 8192, 2048, "float16")),
+    (lambda br, g: _skinny(br, g, 32, 2048, 4096, "float16"), lambda br, g: _skinny(br, g, 64, 8192, 4096, "float16")),
+    (lambda br, g: _transposed_b(br, g, 300), lambda br, g: _transposed_b(br, g, 9000)),
+    (lambda br, g: _conv(br, g, 16), lambda br, g: _conv(br, g, 512))], ids=["f32", "f16", "b", "conv"])
+def test_captured_scratch_outlives_growth(small, large):
+    """Replays after the slot has grown give the eager call's bits, and do not
+    write what took the memory since."""
+    from browsergrad_amd.bridge import HipRealizerBridge
+    rng = np.random.default_rng(11)
+    with HipRealizerBridge(device=0) as br:
+        br.set_profiling(False)
+        fn, grow = small(br, rng), large(br, rng)
+        warm = fn()
+        want = br.to_numpy(warm).copy()
+        br.release(warm)
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=torch.cuda.ExternalStream(br.stream_ptr())):
+            h = fn()
+        eager = br.to_numpy(g := grow()).copy()
+        br.release(g)
+        fill = [br.upload(np.full(1 << 19, 7, F32), (1 << 19,), "float32") for _ in range(16)]
+        for _ in range(3):
+            graph.replay()
+            torch.cuda.synchronize()
+            assert np.array_equal(br.to_numpy(h), want)
+            assert all((br.to_numpy(f) == 7).all() for f in fill)
+            again = grow()
+            assert np.array_equal(br.to_numpy(again), eager)
+            br.release(again)
+        del graph
