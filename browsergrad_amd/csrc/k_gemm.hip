@@ -910,6 +910,12 @@ __global__ void __launch_bounds__(256) gemm_skinny_finish_kernel(GemmArgs P, int
 
 namespace bg {
 
+// Rows of A and B (along K, or along N for a [K][N] B) allow 16-byte loads.
+static bool gemm32_rows_aligned(const bg_matmul_desc& d, bool ptrs_aligned) {
+  return ptrs_aligned && d.lda % 4 == 0 && d.ldb % 4 == 0 && d.k % 4 == 0 && (d.trans_b || d.n % 4 == 0) &&
+         d.stride_a % 4 == 0 && d.stride_b % 4 == 0;
+}
+
 // Launch shape of the f32 GEMM, shared by run_gemm and the launch-plan
 // query.  ptrs_aligned: A and B (offsets applied) start on 16 bytes.
 // Few output tiles and a long K (C1's 64 x 784 x 128): one 128 x 128
@@ -917,12 +923,6 @@ namespace bg {
 // step, so such GEMMs take the wide-K kernel instead (32 x 32 blocks, K
 // split over the wavefronts of a workgroup and summed through LDS, one
 // launch).
-// Rows of A and B (along K, or along N for a [K][N] B) allow 16-byte loads.
-static bool gemm32_rows_aligned(const bg_matmul_desc& d, bool ptrs_aligned) {
-  return ptrs_aligned && d.lda % 4 == 0 && d.ldb % 4 == 0 && d.k % 4 == 0 && (d.trans_b || d.n % 4 == 0) &&
-         d.stride_a % 4 == 0 && d.stride_b % 4 == 0;
-}
-
 Gemm32Shape gemm32_shape(const bg_matmul_desc& d, bool ptrs_aligned) {
   Gemm32Shape g;
   g.tiles_m = int((d.m + 127) / 128);
@@ -961,8 +961,9 @@ static bool gelu_in_epilogue(const bg_matmul_desc& d, const char* a, const char*
 // a / b point at the operands' storage (d.offset_a / d.offset_b are applied
 // here); bias is f32 [N] or NULL.
 // Skinny GEMMs: at most 512 rows for f32 (blocks of 64; above 32 rows only
-// where the product is not split) or 64 for 16-bit, a K of 512+, fewer 128-column tiles than CUs and one batch (the tiled
-// kernels would leave most of the chip idle).
+// where the product is not split) or 64 for 16-bit, a K of 512+, fewer
+// 128-column tiles than CUs and one batch (the tiled kernels would leave most
+// of the chip idle).
 // K slices of at least 256 (and multiples of 64: four wavefronts interleave
 // the steps) until about 256 workgroups stream B; a workspace with less
 // than `room` bytes free for the partials takes one slice.
@@ -979,7 +980,9 @@ static SkinnyPlan skinny_plan(const bg_matmul_desc& d, int dt, size_t room) {
   SkinnyPlan sp;
   sp.ntiles = (d.n + 127) / 128;
   // Row limit: 512 for f32 (64-row blocks; the tiled f32 kernel has at
-  // most 128 workgroups there: 256 x 4096 x 4096 150 against 479 us), 64
+  // most 128 workgroups there: 256 x 4096 x 4096 150 against 479 us; by default
+  // such rows are split, 62 us, so this is the rule of BG_MATMUL_F32_UNSPLIT
+  // and of operands past 2 GiB), 64
   // for 16-bit (two blocks measured slower than the tiled kernel: 50
   // against 40 us at 128 x 4096 x 4096).
   if (d.batch != 1 || d.m > (dt == BG_F32 ? 512 : 64) || d.k < 512 || sp.ntiles >= 256 ||

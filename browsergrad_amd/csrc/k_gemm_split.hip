@@ -331,8 +331,11 @@ Gemm32Split gemm32_split(const bg_matmul_desc& d, bool wide, bool skinny, size_t
   if (d.k <= 4) return g;
   if (skinny && !wide && d.m <= 32 && (!d.trans_b || d.n * d.k <= int64_t(10) << 20)) return g;
   // The wide-K kernel's sizes, first without the model (a few hundred ns of the
-  // call): with up to 32 slices it says at least 9.1 us + k / 730, which is
-  // under 3 us + k / 128 only from k = 940 on.
+  // call).  Up to k = 900: with up to 32 slices the model says at least 9.1 us + k /
+  // 730, which is under 3 us + k / 128 only from k = 940 on.  Outputs of fewer than
+  // 64 x 128 values stay there at any k, as before the split kernel; K slices
+  // would serve long ones better (64 x 64: k = 1200 20.5 us either way, 2000 32.9
+  // against 13.2, 65536 1126 against 103; B as [N][K] 14.4 / 12.4 and 537 / 93).
   if (wide && (d.m * d.n < 64 * 128 || d.k < 900)) return g;
   const int64_t as = ((d.m - 1) * d.lda + d.k) * 4;
   const int64_t bs = (d.trans_b ? (d.n - 1) * d.ldb + d.k : (d.k - 1) * d.ldb + d.n) * 4;
