@@ -229,16 +229,7 @@ namespace bg {
 // four: its tiled kernel is far slower); with four 16-bit rows the vector work
 // costs more than the matrix cores' (8 x 12 heads, 1024 keys: 16.2 against
 // 13.8 us; 32 x 12, 4096 keys: 104 against 79).  From 64 keys: below, the tiled
-// kernels walk one tile.  More heads than CUs keep 16-bit calls on the tiled
-// kernels while the run of keys is short (their workgroups are a quarter of
-// this one's threads) or the heads end in a part of a round of 512 workgroups:
-// one row, f16, tiled against this kernel: 1024 heads, 64 keys 11.1 / 11.5 us, 128
-// 14.1 / 12.5; 320 heads, 128 keys 7.0 / 7.1, 160 7.5 / 6.9; 640 heads, 512 keys
-// 0.96 of the tiled speed, 1536 1.08.  Two rows: 1024 heads, 256 keys 22.4 / 24.1,
-// 384 28.7 / 28.2, 1024 63.6 / 50.7; 512 heads, 1024 keys 24.0 / 28.1.  f32 with
-// more than two rows of 32 columns or fewer: 512 heads of 16, 64 keys 0.81, 65
-// 1.05; 4096 heads of 32, 64 keys 0.96.
-// A workgroup streams about 100 GB/s, so fewer than 64
+// kernels walk one tile.  A workgroup streams about 100 GB/s, so fewer than 64
 // heads with 1 MB of K and V each are cut into slices of 64 KB or more; their
 // second launch costs about 4 us.
 int attention_decode_slices(const bg_attention_desc& d, bool ptrs_aligned) {
@@ -251,11 +242,6 @@ int attention_decode_slices(const bg_attention_desc& d, bool ptrs_aligned) {
   for (int64_t s : {d.q_sb, d.q_sh, d.q_ss, d.k_sb, d.k_sh, d.k_ss, d.v_sb, d.v_sh, d.v_ss})
     if (s % e != 0) return 0;
   const int64_t bh = d.batch * d.heads, bytes = 2 * d.sk * d.d * es;
-  int64_t keys = 64;
-  if (d.in_dtype == BG_F32) keys = d.sq > 2 && d.d <= 32 ? 65 : 64;
-  else if (bh > 256 && d.sq == 1) keys = bh <= 448 ? 129 : bh < 768 ? 1536 : 65;
-  else if (bh > 256) keys = bh < 768 ? INT64_MAX : 384;
-  if (d.sk < keys) return 0;
   if (d.causal || bh >= 64 || bytes < (int64_t(1) << 20)) return 1;
   const int64_t n = std::min<int64_t>(256 / bh, bytes / (int64_t(64) << 10)), ks = (d.sk + n - 1) / n;
   return int((d.sk + ks - 1) / ks);

@@ -78,28 +78,6 @@ def test_decode_attention(bridge, b, h, sq, sk, d, dtype, causal):
         bridge.release(x)
 
 
-@pytest.mark.parametrize("dtype,h,sq,d,keys", [("float16", 256, 1, 8, 64), ("float16", 257, 1, 8, 129),
-                                               ("bfloat16", 449, 1, 8, 1536), ("float16", 768, 1, 8, 65),
-                                               ("float16", 768, 2, 8, 384), ("float32", 300, 3, 16, 65),
-                                               ("float32", 300, 3, 36, 64), ("float32", 300, 2, 16, 64)])
-def test_decode_kernel_choice(bridge, dtype, h, sq, d, keys):
-    """The streaming kernel runs from `keys` keys on, the tiled kernels below; both
-    sides of the edge within the operands' rounding of each other's formula."""
-    rng = np.random.default_rng(h)
-    for sk in (keys - 1, keys):
-        (hq, q), (hk, k), (hv, v) = (_put(bridge, rng.standard_normal((1, h, n, d)).astype(F32), dtype)
-                                     for n in (sq, sk, sk))
-        y, log = _run(bridge, (hq, hk, hv), dtype, batch=1, heads=h, sq=sq, sk=sk, d=d, scale=d ** -0.5)
-        assert all(("attention_decode" in r["kernel"]) == (sk >= keys) for r in log), log
-        s = q @ k.transpose(0, 1, 3, 2) * d ** -0.5
-        p = np.exp(s - s.max(-1, keepdims=True))
-        p /= p.sum(-1, keepdims=True)
-        u = {"float16": 2.0 ** -10, "bfloat16": 2.0 ** -7, "float32": 0.0}[dtype]
-        assert np.all(np.abs(y - p @ v) <= (u + 3e-5) * (p @ np.abs(v)))
-        for x in (hq, hk, hv):
-            bridge.release(x)
-
-
 def test_decode_attention_views_and_rounded_scores(bridge):
     """K and V inside one [B, S, 2, H, D] cache, output [B, Sq, H, D]; and two
     scores that round to one 16-bit value share their weight."""
