@@ -288,6 +288,7 @@ void plan_attention(const bg_attention_desc& d, bg_launch_plan& out);
 // Attention of at most four query rows (k_attn_decode.hip): key slices of the
 // call, 0 where another kernel takes it; launch returns false then.
 int attention_decode_slices(const bg_attention_desc& d, bool ptrs_aligned);
+int attention_decode_waves(const bg_attention_desc& d);  // wavefronts of a workgroup
 bool launch_attention_decode(bg_ctx* ctx, const bg_attention_desc& d, const char* q, const char* k, const char* v,
                              void* o);
 bool fa32_supported(const bg_attention_desc& d);

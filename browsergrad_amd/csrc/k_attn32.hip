@@ -44,6 +44,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstdio>
+#include <initializer_list>
 
 #include "common.cuh"
 #include "core.h"
@@ -714,20 +715,20 @@ void plan_attention(const bg_attention_desc& d0, bg_launch_plan& out) {
     out.tile_n = 1;
     out.tile_k = int32_t(d.d);
     out.k_slices = slices;
-    out.lds_bytes = 16 * nq * 66 * 4;
+    const int waves = attention_decode_waves(d);
+    out.lds_bytes = waves * nq * 66 * 4;
     out.workspace_bytes = slices > 1 ? d.batch * d.heads * slices * d.sq * (d.d + 2) * 4 : 0;
     out.n_launches = slices > 1 ? 2 : 1;
-    auto entry = [&](int i, const char* family, int a0, int a1, int64_t gx, int64_t gy, int threads) {
+    auto entry = [&](int i, const char* family, std::initializer_list<int> targs, int64_t gx, int64_t gy, int threads) {
       bg_launch_plan_entry& e = out.launch[i];
       std::snprintf(e.family, sizeof e.family, "%s", family);
-      e.n_targs = a1 ? 2 : 1;
-      e.targs[0] = a0;
-      e.targs[1] = a1;
+      e.n_targs = int(targs.size());
+      std::copy(targs.begin(), targs.end(), e.targs);
       e.grid[0] = gx; e.grid[1] = gy; e.grid[2] = 1;
       e.block[0] = threads; e.block[1] = 1; e.block[2] = 1;
     };
-    entry(0, "attention_decode_kernel", BG_F32, nq, d.batch * d.heads, slices, 1024);
-    if (slices > 1) entry(1, "attention_decode_merge_kernel", BG_F32, 0, d.batch * d.heads * d.sq, 1, 64);
+    entry(0, "attention_decode_kernel", {BG_F32, nq, waves}, d.batch * d.heads, slices, waves * 64);
+    if (slices > 1) entry(1, "attention_decode_merge_kernel", {BG_F32}, d.batch * d.heads * d.sq, 1, 64);
     return;
   }
   out.tile_m = kBQ;

@@ -2,7 +2,7 @@
 //
 // The MFMA kernels give a workgroup 128 query rows of a (batch, head) and walk
 // its keys tile by tile, so with a row or two they run a serial chain of tiles
-// on a few CUs.  Here one 1024-thread workgroup reads a (batch, head)'s K and V
+// on a few CUs.  Here one workgroup of W wavefronts reads a (batch, head)'s K and V
 // once, every wavefront with four K rows and four V rows of each lane group in
 // flight; a group of 8 (16-bit) or 16 (f32) lanes holds a row, keeps its own
 // running maximum, sum and output, and the groups are merged at the end, inside
@@ -24,7 +24,6 @@ namespace {
 
 using namespace bgk;
 
-constexpr int kDecWaves = 16;
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 struct DecArgs {
@@ -61,14 +60,15 @@ __device__ __forceinline__ float rel_exp2(float a, float b) {
   return __builtin_amdgcn_exp2f(a - (b == -INFINITY ? 0.f : b));
 }
 
-template <int DT, int NQ>
-__global__ void __launch_bounds__(kDecWaves * 64) attention_decode_kernel(DecArgs P) {
+template <int DT, int NQ, int W>
+__global__ void __launch_bounds__(W * 64) attention_decode_kernel(DecArgs P) {
   constexpr int ES = DT == BG_F32 ? 4 : 2;
   constexpr int E = 16 / ES;   // values per lane
   constexpr int L = 64 / E;    // lanes per row
   constexpr int R = 64 / L;    // rows per wavefront load
   constexpr int U = 4;         // rows per lane group in flight
-  __shared__ float red[kDecWaves][NQ][64 + 2];
+  static_assert(W >= NQ, "one wavefront finishes a row");
+  __shared__ float red[W][NQ][64 + 2];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int g = lane / L, c = lane % L;
   const int bh = blockIdx.x, slice = blockIdx.y;
@@ -93,7 +93,7 @@ __global__ void __launch_bounds__(kDecWaves * 64) attention_decode_kernel(DecArg
     l[i] = 0.f;
   }
   const int kall = P.causal ? min(kend, P.Sq) : kend;
-  for (int k0 = kbeg + w * R * U; k0 < kall; k0 += kDecWaves * R * U) {
+  for (int k0 = kbeg + w * R * U; k0 < kall; k0 += W * R * U) {
     u32x4 kr[U], vr[U];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
@@ -176,13 +176,13 @@ __global__ void __launch_bounds__(kDecWaves * 64) attention_decode_kernel(DecArg
   }
   __syncthreads();
   const int i = threadIdx.x >> 6, d = threadIdx.x & 63;
-  if (i >= P.Sq) return;  // Sq <= NQ <= 4 wavefronts
+  if (i >= P.Sq) return;  // Sq <= NQ <= W
   float mm = red[0][i][64];
 #pragma unroll
-  for (int x = 1; x < kDecWaves; ++x) mm = fmaxf(mm, red[x][i][64]);
+  for (int x = 1; x < W; ++x) mm = fmaxf(mm, red[x][i][64]);
   float ls = 0.f, os = 0.f;
 #pragma unroll
-  for (int x = 0; x < kDecWaves; ++x) {
+  for (int x = 0; x < W; ++x) {
     const float f = rel_exp2(red[x][i][64], mm);
     ls += red[x][i][65] * f;
     os += red[x][i][d] * f;
@@ -247,6 +247,24 @@ int attention_decode_slices(const bg_attention_desc& d, bool ptrs_aligned) {
   return int((d.sk + ks - 1) / ks);
 }
 
+// Wavefronts of a workgroup.  Sixteen where a CU has one head, so that all its
+// wavefronts read it; more heads than CUs, or short runs of keys, are better off
+// with workgroups that end sooner (W of them merge through LDS, whatever the run):
+// f16, D64, two rows, 16 / 8 / 4 wavefronts (tiled kernels): 1024 heads, 64 keys
+// 17.7 / 10.7 / 6.5 us (11.1), 256 keys 24.0 / 16.5 / 15.1 (22.2), 1024 keys 50.3 /
+// 42.8 / 42.5 (63.2); 512 heads, 1024 keys 28.0 / 24.2 / 24.0 (23.9); 96 heads, 192
+// keys 6.5 / 6.2 / 6.2 (6.2), 1024 keys 10.8 / 11.2 / 13.4 (14.1).  One row: 1024
+// heads, 64 keys 11.3 / 7.2 / 6.1 (11.0).  A float32 wavefront takes half the keys
+// a step, so its runs are short up to 128 keys, and fewer than eight serve none
+// but three and four rows: one row, D24, 272 heads, 512 keys 7.9 / - / 9.2 us; D64,
+// 4096 heads, 128 keys 42.3 / 38.9 / 39.1; four rows, 272 heads, 64 keys 9.5 / 6.2
+// / 6.2 (14.7), 1024 heads, 1024 keys 102 / 94 / 95 (292).
+int attention_decode_waves(const bg_attention_desc& d) {
+  const bool many = d.batch * d.heads > 256;
+  if (d.in_dtype == BG_F32) return (many && d.sq > 2) || d.sk <= 128 ? 8 : 16;
+  return many ? 4 : d.sk <= 512 ? 8 : 16;
+}
+
 bool launch_attention_decode(bg_ctx* ctx, const bg_attention_desc& d, const char* q, const char* k, const char* v,
                              void* o) {
   auto al16 = [](const char* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
@@ -275,16 +293,25 @@ bool launch_attention_decode(bg_ctx* ctx, const bg_attention_desc& d, const char
   A.ks = int((d.sk + slices - 1) / slices);
   if (A.slices > 1) A.part = static_cast<float*>(scratch(ctx, size_t(bh * A.slices * d.sq * (d.d + 2)) * 4, 3));
   const dim3 grid(unsigned(bh), unsigned(A.slices));
-  auto by_q = [&](auto dt) {
-    constexpr int DT = decltype(dt)::value;
-    if (d.sq == 1) dispatch(ctx, attention_decode_kernel<DT, 1>, grid, dim3(kDecWaves * 64), 0, A);
-    else if (d.sq == 2) dispatch(ctx, attention_decode_kernel<DT, 2>, grid, dim3(kDecWaves * 64), 0, A);
-    else if constexpr (DT == BG_F32) dispatch(ctx, attention_decode_kernel<DT, 4>, grid, dim3(kDecWaves * 64), 0, A);
+  auto by_q = [&](auto dt, auto waves) {
+    constexpr int DT = decltype(dt)::value, W = decltype(waves)::value;
+    if constexpr (DT != BG_F32 || W > 4) {
+      if (d.sq == 1) dispatch(ctx, attention_decode_kernel<DT, 1, W>, grid, dim3(W * 64), 0, A);
+      else if (d.sq == 2) dispatch(ctx, attention_decode_kernel<DT, 2, W>, grid, dim3(W * 64), 0, A);
+      else if constexpr (DT == BG_F32) dispatch(ctx, attention_decode_kernel<DT, 4, W>, grid, dim3(W * 64), 0, A);
+    }
     if (A.part) dispatch(ctx, attention_decode_merge_kernel<DT>, dim3(unsigned(bh * d.sq)), dim3(64), 0, A);
   };
-  if (d.in_dtype == BG_F32) by_q(std::integral_constant<int, BG_F32>{});
-  else if (d.in_dtype == BG_F16) by_q(std::integral_constant<int, BG_F16>{});
-  else by_q(std::integral_constant<int, BG_BF16>{});
+  auto by_waves = [&](auto dt) {
+    switch (attention_decode_waves(d)) {
+      case 4: by_q(dt, std::integral_constant<int, 4>{}); break;
+      case 8: by_q(dt, std::integral_constant<int, 8>{}); break;
+      default: by_q(dt, std::integral_constant<int, 16>{});
+    }
+  };
+  if (d.in_dtype == BG_F32) by_waves(std::integral_constant<int, BG_F32>{});
+  else if (d.in_dtype == BG_F16) by_waves(std::integral_constant<int, BG_F16>{});
+  else by_waves(std::integral_constant<int, BG_BF16>{});
   return true;
 }
 

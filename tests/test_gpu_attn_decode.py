@@ -78,6 +78,36 @@ def test_decode_attention(bridge, b, h, sq, sk, d, dtype, causal):
         bridge.release(x)
 
 
+# Heads on both sides of one a CU, runs of keys on both sides of a step of four
+# and eight wavefronts (32 16-bit or 16 float32 rows each) and of the 512 rule.
+@pytest.mark.parametrize("h,sk,waves", [(256, 64, 8), (5, 255, 8), (5, 257, 8), (256, 512, 8), (256, 513, 16),
+                                        (257, 64, 4), (300, 127, 4), (300, 129, 4), (257, 513, 4), (5, 129, 8)])
+@pytest.mark.parametrize("dtype,sq", [("float16", 1), ("bfloat16", 2), ("float32", 1), ("float32", 3)])
+def test_decode_wavefronts(bridge, h, sk, waves, dtype, sq):
+    if dtype == "float32":
+        waves = 8 if h > 256 and sq > 2 or sk <= 128 else 16
+    d = 24
+    rng = np.random.default_rng(sk)
+    (hq, q), (hk, k), (hv, v) = (_put(bridge, rng.standard_normal((1, h, n, d)).astype(F32), dtype)
+                                 for n in (sq, sk, sk))
+    y, log = _run(bridge, (hq, hk, hv), dtype, batch=1, heads=h, sq=sq, sk=sk, d=d, scale=d ** -0.5)
+    assert len(log) == 1 and "attention_decode_kernel" in log[0]["kernel"] and log[0]["block"][0] == 64 * waves
+    if dtype == "float32":
+        from browsergrad_amd.semantic import launch_plan
+        a = N.AttentionDesc()
+        a.batch, a.heads, a.sq, a.sk, a.d = 1, h, sq, sk, d
+        a.in_dtype = a.out_dtype = N.BG_F32
+        assert [(r["grid"], r["block"]) for r in log] == [(e["grid"], e["block"])
+                                                         for e in launch_plan("attention", a)["launches"]]
+    s = q @ k.transpose(0, 1, 3, 2) * d ** -0.5
+    p = np.exp(s - s.max(-1, keepdims=True))
+    p /= p.sum(-1, keepdims=True)
+    u = {"float16": 2.0 ** -11, "bfloat16": 2.0 ** -8, "float32": 0.0}[dtype]
+    assert np.all(np.abs(y - p @ v) <= (u + 3e-5) * (p @ np.abs(v)))
+    for x in (hq, hk, hv):
+        bridge.release(x)
+
+
 def test_decode_attention_views_and_rounded_scores(bridge):
     """K and V inside one [B, S, 2, H, D] cache, output [B, Sq, H, D]; and two
     scores that round to one 16-bit value share their weight."""
