@@ -379,8 +379,8 @@ __global__ void __launch_bounds__(256) conv_gemm_kernel(ConvK P) {
 //
 // Bound by x's gathers (a load's 64 lanes touch about seven channels' three
 // rows) beside the matrix core.  Measured, with the sum over the slices: 32 x
-// 128 x 28 x 28 with 128 3x3 filters 115 -> 73 us (its 44 GFLOP of bf16
-// products take 37 us at 1.2 PFLOP/s), 32 x 64 x 56 x 56 163 -> 112, 64 x 256 x
+// 128 x 28 x 28 with 128 3x3 filters 107 -> 70 us (its 44 GFLOP of bf16
+// products take 37 us at 1.2 PFLOP/s), 32 x 64 x 56 x 56 162 -> 107, 64 x 256 x
 // 14 x 14 204 -> 154; error against 64 bits 3.5e-7 -> 1.8e-7.
 template <int BM, int WGM, int WGN>
 __global__ void __launch_bounds__(256, 2)

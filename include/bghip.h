@@ -409,10 +409,11 @@ int bg_matmul_ex2(bg_ctx* ctx, const bg_matmul_desc* desc, const bg_matmul_ext* 
  * ldc, strides as in bg_matmul_ex, ldc / stride_c 0 = contiguous), the
  * caller sizes them (no extent check is possible), and the call allocates
  * nothing: no handle, no profiling event, and the kernels' scratch comes
- * from a fixed 16 MiB array per GPU held until the process ends.  Problems
- * that need more scratch (split-K partials of long-K f32 GEMMs, the
- * re-laid-out B of x @ w, the f32 product before a separate GELU pass) are
- * refused with BG_E_UNSUPPORTED before anything is launched.  The array is
+ * from a fixed 16 MiB array per GPU held until the process ends.  K-slice
+ * partials take what room it has: fewer slices, or one.  Problems that need
+ * more for a re-laid-out B of x @ w, a cast operand or the f32 product before
+ * a separate GELU pass are refused with BG_E_UNSUPPORTED before anything is
+ * launched.  The array is
  * shared by every call on one GPU: calls that overlap on one GPU (different
  * contexts or threads) race; calls on one context are stream ordered. */
 int bg_matmul_noalloc(bg_ctx* ctx, const bg_matmul_desc* desc, const void* a, const void* b,

@@ -183,7 +183,7 @@ def test_split_attention_small_weights(bridge):
 
 @pytest.mark.parametrize("what", ["nan_k", "inf_v", "neg_inf_k", "tiny_v", "tiny_k", "huge_q"])
 def test_split_attention_special_values(bridge, what):
-    """What the parts cannot hold gives what the float32 kernel gives."""
+    """What the parts cannot hold, and tiny values, give what the float32 kernel gives."""
     rng = np.random.default_rng(8)
     b, h, s, d = 1, 2, 140, 64
     q, k, v = (rng.standard_normal((b, h, s, d)).astype(F32) for _ in range(3))

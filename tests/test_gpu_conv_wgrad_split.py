@@ -97,8 +97,8 @@ def test_small_values_take_no_other_path(bridge, e, o):
 
 @pytest.mark.parametrize("value", [2.0**-120, 1e-40, np.inf, np.nan, 3.4e38])
 def test_values_the_parts_cannot_hold(bridge, value):
-    """A dy value below 2^-109, infinite, NaN or one whose leading part rounds to
-    infinity: the workgroup's float32 sums give what float32 gives."""
+    """A dy value infinite, NaN or one whose leading part rounds to infinity (the
+    workgroup's float32 sums), or a tiny one, gives what float32 gives."""
     geo = ((3, 3), (1, 1), (1, 1), (1, 1))
     x, dy = _data(2, 16, 40, (10, 10), *geo, False, 5)
     x = np.abs(x) + F32(1)
