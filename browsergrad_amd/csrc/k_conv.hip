@@ -372,16 +372,17 @@ __global__ void __launch_bounds__(256) conv_gemm_kernel(ConvK P) {
 // three 16-deep stages, the two sets of sums and the float32 redo are those of
 // gemm32_split_kernel; both operands pass through registers here.  dy: lanes
 // 2 r and 2 r + 1 read eight consecutive positions of row r each (two 16-byte
-// loads where an image holds a multiple of eight).  x: the 64 columns (c, tap)
-// of a wavefront take the same eight positions, which the scalar unit
-// decomposes; they end at most one row (oW >= 8), so a column keeps the offsets
-// of two rows and adds its position's.
+// loads where an image holds a multiple of four; by single loads 32 x 128 x 28 x
+// 28 with 16 1x1 filters of stride 2 took 22.1 us, 19.7 on the float32 kernel and
+// 20.4 so).  x: the 64 columns (c, tap) of a wavefront take the same eight
+// positions, which the scalar unit decomposes; they end at most one row (oW >=
+// 8), so a column keeps the offsets of two rows and adds its position's.
 //
 // Bound by x's gathers (a load's 64 lanes touch about seven channels' three
 // rows) beside the matrix core.  Measured, with the sum over the slices: 32 x
 // 128 x 28 x 28 with 128 3x3 filters 107 -> 70 us (its 44 GFLOP of bf16
 // products take 37 us at 1.2 PFLOP/s), 32 x 64 x 56 x 56 162 -> 107, 64 x 256 x
-// 14 x 14 204 -> 154; error against 64 bits 3.5e-7 -> 1.8e-7.
+// 14 x 14 197 -> 118; error against 64 bits 3.5e-7 -> 1.8e-7.
 template <int BM, int WGM, int WGN>
 __global__ void __launch_bounds__(256, 2)
     conv_wgrad_split_kernel(ConvK P, uint32_t a_bytes, uint32_t b_bytes, int a16) {
@@ -434,10 +435,12 @@ __global__ void __launch_bounds__(256, 2)
       const uint32_t n = fdiv(k, P.f_oS), sp = k - n * uint32_t(P.oS);
       const uint32_t off = a_row + (n * uint32_t(P.O) * uint32_t(P.oS) + sp) * 4;
       if (a16) {
-        const uint32_t at = off | (a_row & kOut) | (int(k) < kend ? 0u : kOut);
+        // (The second four positions may be the next image's first.)
+        const uint32_t next = off + 16u + (sp + 4u == uint32_t(P.oS) ? uint32_t((P.O - 1) * P.oS) * 4u : 0u);
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
-          const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(ra, at + 16 * h, 0, 0);
+          const uint32_t at = (h ? next : off) | (a_row & kOut) | (int(k) + 4 * h < kend ? 0u : kOut);
+          const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(ra, at, 0, 0);
 #pragma unroll
           for (int e = 0; e < 4; ++e) xa[4 * h + e] = __uint_as_float(v[e]);
         }
@@ -546,12 +549,12 @@ __global__ void __launch_bounds__(256, 2)
         __builtin_amdgcn_s_barrier();
         // (With four tiles a wavefront the branch keeps the split behind the barrier:
         // its first multiplies, moved before it, wait for the stage's loads, 1 x 256 x
-        // 64 x 64 with 256 filters 58.1 -> 54.6 us.  With two they wait less than the
+        // 64 x 64 with 256 filters 58.1 -> 55.3 us.  With two they wait less than the
         // lost overlap costs: 32 x 64 x 56 x 56 107.0, with the branch 114.7.)
         if (more) put_a(wslot);
       }
       if (i == 1) {
-        if (more) put_b(wslot);
+        put_b(wslot);
         load_stage(t + 3);
       }
     }
@@ -1381,7 +1384,7 @@ void launch_conv(bg_ctx* ctx, const ConvProblem& p, int mode, const float* a, co
   const dim3 grid(unsigned(tiles), unsigned(G * k.ksplit));
   if (wsplit) {
     const uint32_t ab = uint32_t(p.n * int64_t(k.O) * k.oS * 4), bb = uint32_t(p.n * int64_t(k.C) * k.S * 4);
-    const int a16 = k.oS % 8 == 0 && (reinterpret_cast<uintptr_t>(a) & 15) == 0;
+    const int a16 = k.oS % 4 == 0 && (reinterpret_cast<uintptr_t>(a) & 15) == 0;
     auto go = [&](auto kern) { dispatch(ctx, kern, grid, dim3(256), 0, k, ab, bb, a16); };
     bm == 128 ? go(conv_wgrad_split_kernel<128, 2, 2>) : go(conv_wgrad_split_kernel<64, 1, 4>);
     if (k.ksplit > 1)

@@ -57,6 +57,9 @@ def _data(n, c, o, size, kernel, stride, pad, dil, transposed, seed):
 CASES = [
     (2, 16, 130, (8, 8), (3, 3), (1, 1), (1, 1), (1, 1), 1, False),     # chunks end with rows; two row tiles
     (3, 15, 70, (9, 9), (3, 3), (1, 1), (1, 1), (1, 1), 1, False),      # odd image: dy element by element
+    (5, 32, 70, (14, 14), (2, 2), (1, 1), (0, 1), (1, 1), 1, False),    # 13 x 15: dy element by element
+    (6, 140, 70, (14, 14), (1, 1), (1, 1), (0, 0), (1, 1), 1, False),   # 196: a chunk's halves in two images
+    (3, 140, 20, (6, 10), (1, 1), (1, 1), (0, 0), (1, 1), 1, False),    # 60 positions, two row groups
     (2, 16, 3, (13, 11), (3, 3), (1, 1), (1, 1), (1, 1), 1, False),     # few rows
     (4, 64, 128, (28, 28), (3, 3), (2, 2), (1, 1), (1, 1), 1, False),   # stride
     (2, 40, 64, (16, 12), (2, 3), (1, 1), (0, 2), (2, 2), 1, False),    # dilation, uneven padding
